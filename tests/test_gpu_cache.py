@@ -88,3 +88,52 @@ def test_out_of_pool_slots_skipped(dev):
     rk, rv = kc.copy(), vc.copy()
     oracle.reshape_and_cache(key, value, rk, rv, keep)
     assert np.array_equal(gk.view(np.uint16), rk.view(np.uint16))
+
+
+def _runs(rng, T, NB, BS=16):
+    """T slots in runs of 1-20 consecutive ones that start anywhere in a block
+    and stop at its end; a few padded (-1) or past the pool."""
+    slots = []
+    for b in rng.permutation(NB):
+        if len(slots) >= T:
+            break
+        o = int(rng.integers(0, BS)) if rng.random() < 0.5 else 0
+        n = int(min(rng.integers(1, 21), BS - o))
+        slots += [int(b) * BS + o + i for i in range(n)]
+    slots = np.array(slots[:T], np.int32)
+    assert len(slots) == T
+    bad = rng.random(T) < 0.03
+    slots[bad] = rng.choice([-1, -16, NB * BS, NB * BS + 5], size=int(bad.sum()))
+    return slots
+
+
+@pytest.mark.parametrize("T,Hkv,D,offset", [
+    (1, 8, 128, 0), (3, 8, 64, 0), (17, 1, 16, 0), (64, 3, 80, 0),
+    (511, 8, 64, 0), (512, 2, 128, 0), (513, 2, 128, 0),   # both window sizes
+    (1037, 5, 80, 0),                                      # a partial last slice of rows
+    (300, 8, 64, 2), (40, 3, 72, 2), (700, 8, 64, 8),      # the token kernel: alignment, rows
+    (200, 1, 40, 0),
+])
+def test_runs_of_slots_bit_exact(dev, T, Hkv, D, offset):
+    """Whole blocks, partial runs, lone and skipped tokens in one call; key and
+    value `offset` bytes past a 16-byte boundary."""
+    rng = np.random.default_rng(T + 31 * D)
+    BS, NB = 16, T + 4
+    slots = _runs(rng, T, NB)
+    key = rng.standard_normal((T, Hkv, D)).astype(np.float16)
+    value = rng.standard_normal((T, Hkv, D)).astype(np.float16)
+    kc = np.full((NB, Hkv, D, BS), SENTINEL, np.uint16).view(np.float16)
+    bufs = []
+    for x in (key, value):
+        buf = DeviceArray((x.size + 8,), np.float16)
+        buf.upload_at(offset, x)
+        bufs.append(buf)
+    kc_d, vc_d, s_d = DeviceArray.from_numpy(kc), DeviceArray.from_numpy(kc), DeviceArray.from_numpy(slots)
+    pa.launch_reshape_and_cache(bufs[0].ptr + offset, bufs[1].ptr + offset, kc_d, vc_d, s_d, T,
+                                Hkv, D, BS, num_blocks=NB)
+    synchronize()
+    keep = np.where((slots >= 0) & (slots < NB * BS), slots, -1).astype(np.int32)
+    rk, rv = kc.copy(), kc.copy()
+    oracle.reshape_and_cache(key, value, rk, rv, keep)
+    assert np.array_equal(kc_d.numpy().view(np.uint16), rk.view(np.uint16))
+    assert np.array_equal(vc_d.numpy().view(np.uint16), rv.view(np.uint16))
