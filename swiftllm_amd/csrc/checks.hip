@@ -5,8 +5,8 @@
 //   max_over_kg / sum_over_kg (attention_core.hpp): lanes l, l ^ 16, l ^ 32,
 //       l ^ 48 on the permlane16/32 swaps (the softmax row max and sum of
 //       the MFMA accumulator layout, decode and prefill);
-//   wave_max / wave_sum (common.hpp): all 64 lanes by xor shuffles (the
-//       split-K reduce);
+//   wave_max / wave_sum (common.hpp): all 64 lanes by DPP moves (the split-K
+//       reduce);
 //   wave_inclusive_scan (common.hpp): the 64-lane prefix sum (MoE dispatch,
 //       split-K item lists).
 // The functions run here are the ones the kernels inline, not copies.
@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256) void wave_reduce_check_kernel(const ReduceChec
     o[128 + lane] = wave_max(v);
     o[192 + lane] = wave_sum(v);
     a.scan[static_cast<size_t>(row) * 64 + lane] =
-        wave_inclusive_scan(a.xi[static_cast<size_t>(row) * 64 + lane], lane);
+        wave_inclusive_scan(a.xi[static_cast<size_t>(row) * 64 + lane]);
 }
 
 }  // namespace

@@ -95,29 +95,52 @@ __host__ __device__ inline int kv_elem_offset(int d, int t) {
 }
 
 // ---------------------------------------------------------------------------
-// Whole-wave reductions (wave64). Every lane ends with the same value; the
-// butterfly adds pairs in the same order in every lane.
+// Whole-wave reductions (wave64), on DPP moves: shifts by 1, 2, 4 and 8 inside
+// the rows of 16 lanes, then the last lane of rows 0 and 2 broadcast into rows
+// 1 and 3, then lane 31 into rows 2 and 3. Six VALU operations, where shuffles
+// are six trips through the LDS crossbar. All 64 lanes must be active. Lane 63
+// ends with the whole wave's value (a balanced tree of depth 6); a maximum or
+// a sum is broadcast from it, so every lane has the same bits.
 // ---------------------------------------------------------------------------
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp(int old, int x) {
+    return __builtin_amdgcn_update_dpp(old, x, CTRL, ROWS, 0xf, false);
+}
+// x combined with its DPP-moved self at each of the six steps; lanes that a
+// step moves nothing into combine with `none`.
+template <typename Op>
+__device__ __forceinline__ int dpp_scan(int x, int none, Op op) {
+    x = op(x, dpp<0x111, 0xf>(none, x));  // row_shr:1
+    x = op(x, dpp<0x112, 0xf>(none, x));
+    x = op(x, dpp<0x114, 0xf>(none, x));
+    x = op(x, dpp<0x118, 0xf>(none, x));
+    x = op(x, dpp<0x142, 0xa>(none, x));  // row_bcast:15
+    x = op(x, dpp<0x143, 0xc>(none, x));  // row_bcast:31
+    return x;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-    return v;
+    const int r = dpp_scan(__builtin_bit_cast(int, v), __builtin_bit_cast(int, -INFINITY), [](int a, int b) {
+        return __builtin_bit_cast(int, fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)));
+    });
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(r, 63));
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
+    const int r = dpp_scan(__builtin_bit_cast(int, v), 0, [](int a, int b) {
+        return __builtin_bit_cast(int, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b));
+    });
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(r, 63));
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave.
-__device__ __forceinline__ int wave_inclusive_scan(int x, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d);
-        if (lane >= d) x += y;
-    }
-    return x;
+__device__ __forceinline__ int wave_inclusive_scan(int x) {
+    return dpp_scan(x, 0, [](int a, int b) { return a + b; });
+}
+
+// The sum of x over the wave.
+__device__ __forceinline__ int wave_total(int x) {
+    return __builtin_amdgcn_readlane(wave_inclusive_scan(x), 63);
 }
 
 }  // namespace swiftllm

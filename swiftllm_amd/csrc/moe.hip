@@ -7,18 +7,25 @@
 // (crates/swiftllm-core/src/sampling/mod.rs:380-385) and ranking is a stable
 // descending sort, so equal logits keep the lower index first (:367-377).
 //
-// route:    one thread per token; K argmax passes over the E logits (value
-//           descending, ties to the lower index), then weights
+// route:    the K largest of the E logits (value descending, ties to the
+//           lower index), then weights
 //           w_k = exp(x_k - x_max) / sum_k' exp(x_k' - x_max), which equals the
 //           softmax probabilities renormalised over the selected experts, in
-//           fp32. Rows of up to 8 or 16 logits are loaded into registers at
-//           once.
+//           fp32. Up to 16 experts: one thread per token, the row in
+//           registers, K argmax passes. More: 16 lanes per token, the row
+//           spread over them, each pass a maximum and an index over the lanes
+//           by DPP. One thread per token re-read its row from memory K times:
+//           route and dispatch of 1000 tokens over 64 experts, top-8, hidden
+//           2048, took 130 us and take 19.2; of 4096 tokens, top-6, 121 and
+//           29.7 (100 MB of rows at 5.7 TB/s of copy: 20).
 // dispatch: two kernels, with no grid-wide synchronisation inside either.
-//           (1) rank: one wave per 64-token chunk ranks the chunk's entries
-//               among equal experts with ballots (stable (t, k) order; for up
-//               to 16 experts one unrolled pass of ballots and mbcnt per
-//               expert) and stores per-(chunk, expert) counts. The fused entry point routes
-//               the chunk's tokens first, in the same wave.
+//           (1) rank: the entries of each 64-token chunk get their rank among
+//               equal experts (stable (t, k) order) and the chunk its counts
+//               per expert. Up to 16 experts: one wave per chunk, an unrolled
+//               pass of ballots and mbcnt per expert. More: one workgroup per
+//               chunk, a 64-bit mask of tokens per expert in LDS. The fused
+//               entry point routes the chunk's tokens first, in the same
+//               kernel.
 //           (2) permute: each workgroup scans the chunk counts (up to 4096
 //               of them) in LDS into per-(chunk, expert) prefixes and expert
 //               offsets, while the first loads of its rows are in flight.
@@ -142,6 +149,78 @@ __device__ __forceinline__ void select_topk(const float* row, int E, float (&bv)
     }
 }
 
+// Top-K of one row of logits by the 16 lanes of a DPP row, for E > 16: lane j
+// holds logits j, j + 16, ... (N of them at most) as integers in the logits'
+// order, and K passes each take the row's maximum and then the lowest index
+// that has it, two chains of four DPP steps. Every lane of the row ends with
+// the K picks. Requires logits without NaN; `row` is null for rows past T.
+__device__ __forceinline__ int ordered(float x) {
+    const int b = __builtin_bit_cast(int, x + 0.0f);  // -0 ranks as 0
+    return b ^ ((b >> 31) & 0x7fffffff);
+}
+template <int CTRL>
+__device__ __forceinline__ int row_ror(int x) {
+    return __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false);
+}
+__device__ __forceinline__ int row_max(int x) {
+    x = max(x, row_ror<0x121>(x));
+    x = max(x, row_ror<0x122>(x));
+    x = max(x, row_ror<0x124>(x));
+    return max(x, row_ror<0x128>(x));
+}
+
+template <int K, int N>
+__device__ __forceinline__ void select_topk_row(const float (&v)[N], int E, int j, float (&bv)[K], int (&bi)[K]) {
+    constexpr int kTaken = INT_MIN;  // below every logit's key, -inf included
+    int key[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) key[i] = (16 * i + j < E) ? ordered(v[i]) : kTaken;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        int best = key[0];
+#pragma unroll
+        for (int i = 1; i < N; ++i) best = max(best, key[i]);
+        best = row_max(best);
+        int first = INT_MIN;  // minus the lowest index
+#pragma unroll
+        for (int i = N - 1; i >= 0; --i) first = (key[i] == best) ? -(16 * i + j) : first;
+        const int e = -row_max(first);
+#pragma unroll
+        for (int i = 0; i < N; ++i) key[i] = (16 * i + j == e) ? kTaken : key[i];
+        bi[k] = e;
+        bv[k] = __builtin_bit_cast(float, best ^ ((best >> 31) & 0x7fffffff));
+    }
+}
+
+// Routes token t (16 lanes per token, j the lane's place) for E > 16: ids in
+// bi, and ids and weights written by the row's first lanes. A wave that holds
+// a NaN routes with the one-thread selection, whose order then counts.
+template <int K, int N>
+__device__ __forceinline__ void route_row(const RouteArgs& a, int t, int j, int (&bi)[K]) {
+    const bool live = t < a.T;
+    const float* row = a.logits + static_cast<size_t>(min(t, a.T - 1)) * a.E;
+    float v[N];
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        v[i] = row[min(16 * i + j, a.E - 1)];
+        nan = nan || !(v[i] == v[i]);
+    }
+    float bv[K];
+    if (__any(nan)) {
+        select_topk<K, 16>(row, a.E, bv, bi);
+    } else {
+        select_topk_row<K, N>(v, a.E, j, bv, bi);
+    }
+    if (live && j == 0) write_route<K>(a, t, bv, bi);
+}
+
+template <int K, int N>
+__global__ __launch_bounds__(256) void moe_route_wide_kernel(const RouteArgs a) {
+    int bi[K];
+    route_row<K, N>(a, blockIdx.x * 16 + (threadIdx.x >> 4), threadIdx.x & 15, bi);
+}
+
 template <int K, int R>
 __global__ __launch_bounds__(256) void moe_route_kernel(const RouteArgs a) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -257,14 +336,10 @@ constexpr int kRankWaves = 4;
 
 template <int K, int R>
 __global__ __launch_bounds__(64 * kRankWaves) void moe_rank_kernel(const RankArgs a) {
-    __shared__ int s_cnt[kRankWaves][kMaxExperts];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
     const int c = blockIdx.x * kRankWaves + wv;  // chunk of this wave
     if (c >= a.nchunks) return;                   // whole waves only; no barriers below
-    if (a.E > kRankUnrolled) {
-        for (int e = lane; e < a.E; e += 64) s_cnt[wv][e] = 0;
-    }
 
     const int t = c * kChunkTokens + lane;
     const bool live = t < a.T;
@@ -283,23 +358,89 @@ __global__ __launch_bounds__(64 * kRankWaves) void moe_rank_kernel(const RankArg
 #pragma unroll
         for (int k = 0; k < K; ++k) id[k] = live ? a.ids[static_cast<size_t>(t) * K + k] : -1;
     }
-    if (a.E <= kRankUnrolled) {
-        int cnt;
-        rank_chunk_unrolled<K>(id, rk, a.E, lane, cnt);
-        if (live) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) a.rank[static_cast<size_t>(t) * K + k] = rk[k];
-        }
-        if (lane < a.E) a.cnt[static_cast<size_t>(c) * a.E + lane] = cnt;
-        return;
-    }
-    rank_chunk<K>(id, rk, a.E, lane, s_cnt[wv]);
+    int cnt;
+    rank_chunk_unrolled<K>(id, rk, a.E, lane, cnt);
     if (live) {
 #pragma unroll
         for (int k = 0; k < K; ++k) a.rank[static_cast<size_t>(t) * K + k] = rk[k];
     }
-    // LDS operations of one wave complete in order: lane 0's counts are seen.
-    for (int e = lane; e < a.E; e += 64) a.cnt[static_cast<size_t>(c) * a.E + e] = s_cnt[wv][e];
+    if (lane < a.E) a.cnt[static_cast<size_t>(c) * a.E + lane] = cnt;
+}
+
+// The rank kernel for E > 16: one workgroup of 16 waves per 64-token chunk, 16
+// lanes per token. With logits each token is routed first. Every entry sets
+// its token's bit in its expert's 64-bit mask in LDS; an entry's rank is the
+// number of lower tokens in the mask, a count the whole mask (the K experts of
+// a routed token differ). Caller-given ids may repeat inside a token: such a
+// chunk is ranked by one wave with the general rounds.
+constexpr int kWideThreads = 16 * kChunkTokens;
+
+template <int K, int N>
+__global__ __launch_bounds__(kWideThreads) void moe_rank_wide_kernel(const RankArgs a) {
+    __shared__ unsigned s_mask[kMaxExperts][2];
+    __shared__ int s_id[kChunkTokens][K];
+    __shared__ int s_cnt[kMaxExperts];
+    const int c = blockIdx.x;
+    const int tok = threadIdx.x >> 4;
+    const int j = threadIdx.x & 15;
+    const int t = c * kChunkTokens + tok;
+    const bool live = t < a.T;
+    for (int e = threadIdx.x; e < a.E; e += kWideThreads) {
+        s_mask[e][0] = s_mask[e][1] = 0u;
+        s_cnt[e] = 0;
+    }
+    int id[K];
+    if (a.logits != nullptr) {
+        route_row<K, N>(RouteArgs{a.logits, a.ids, a.w, a.T, a.E}, t, j, id);
+    } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) id[k] = a.ids[static_cast<size_t>(min(t, a.T - 1)) * K + k];
+    }
+    bool twice = false;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (!live || id[k] < 0 || id[k] >= a.E) id[k] = -1;
+#pragma unroll
+        for (int k2 = 0; k2 < k; ++k2) twice = twice || (id[k] >= 0 && id[k] == id[k2]);
+    }
+    const bool repeats = __syncthreads_or(twice);  // also: the masks are clear
+    if (j == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) s_id[tok][k] = id[k];
+    }
+    int mine = -1;  // lane j < K owns entry (t, j)
+#pragma unroll
+    for (int k = 0; k < K; ++k) mine = (j == k) ? id[k] : mine;
+    if (mine >= 0) atomicOr(&s_mask[mine][tok >> 5], 1u << (tok & 31));
+    __syncthreads();
+    if (repeats) {
+        if (threadIdx.x < 64) {
+            const int lane = threadIdx.x;
+            int rk[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) id[k] = s_id[lane][k];
+            rank_chunk<K>(id, rk, a.E, lane, s_cnt);
+            if (c * kChunkTokens + lane < a.T) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) a.rank[static_cast<size_t>(c * kChunkTokens + lane) * K + k] = rk[k];
+            }
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < a.E; e += kWideThreads) a.cnt[static_cast<size_t>(c) * a.E + e] = s_cnt[e];
+        return;
+    }
+    if (live && j < K) {
+        int rk = -1;
+        if (mine >= 0) {
+            const unsigned lo = s_mask[mine][0], hi = s_mask[mine][1];
+            const unsigned below = (1u << (tok & 31)) - 1u;
+            rk = tok < 32 ? __popc(lo & below) : __popc(lo) + __popc(hi & below);
+        }
+        a.rank[static_cast<size_t>(t) * K + j] = rk;
+    }
+    for (int e = threadIdx.x; e < a.E; e += kWideThreads) {
+        a.cnt[static_cast<size_t>(c) * a.E + e] = __popc(s_mask[e][0]) + __popc(s_mask[e][1]);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -327,7 +468,7 @@ __global__ __launch_bounds__(kScanThreads) void moe_scan_kernel(const ScanArgs a
     const int c1 = min(c0 + per, a.nchunks);
     int sum = 0;
     for (int c = c0; c < c1; ++c) sum += a.cnt[static_cast<size_t>(c) * a.E + e];
-    const int x = wave_inclusive_scan(sum, lane);
+    const int x = wave_inclusive_scan(sum);
     if (lane == 63) s_wave[wv] = x;
     __syncthreads();
     int run = x - sum;
@@ -354,6 +495,15 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kCopyBatch = 8;          // 16-byte loads per lane in flight before the stores
 constexpr int kPermuteWaves = 4;       // one token per wave
 constexpr int kLdsCounts = 4096;       // count matrices up to this size are scanned in LDS
+constexpr int kLdsPad = 512;           // room for one more column (E >= 8)
+
+// Bytes of x_perm up to which its rows are stored nontemporally. Past it the
+// caches take the writes and return them in larger pieces; below it the dirty
+// lines they hold are written back at the kernel's end instead. Measured (us
+// per call, 8 experts, top-2, nontemporal / plain): 67 MB of rows 20.5 / 19.3,
+// 47.5 MB 15.3 / 15.3, 32.8 MB 11.8 / 12.9, 16.4 MB 8.6 / 9.7; 64 experts,
+// top-6, 100 MB 31.1 / 29.7.
+constexpr size_t kNontemporalRows = 48u << 20;
 
 struct PermuteArgs {
     const int* ids;
@@ -375,10 +525,11 @@ struct PermuteArgs {
 };
 
 // VEC: rows move as 16-byte vectors (a.xp set and a.vec); otherwise index
-// arrays only, or a 2-byte copy of unaligned rows.
-template <int K, bool VEC>
+// arrays only, or a 2-byte copy of unaligned rows. NT: nontemporal stores of
+// the rows.
+template <int K, bool VEC, bool NT>
 __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const PermuteArgs a) {
-    __shared__ int s_base[kLdsCounts];  // [nchunks][E] exclusive prefixes over chunks
+    __shared__ int s_base[kLdsCounts + kLdsPad];  // [nchunks][stride] exclusive prefixes over chunks
     __shared__ int s_off[kMaxExperts];  // expert offsets
     if (a.T == 0) {
         // No tokens (one workgroup): zero counts and offsets. Below, T >= 1,
@@ -403,6 +554,10 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
     // wait for all of them before the first count is used.
     constexpr int kCntPerThread = kLdsCounts / (64 * kPermuteWaves);
     const int n = a.nchunks * a.E;
+    // The scans walk a column of the counts; for a power of two of experts the
+    // rows are one longer in LDS, or its entries would share a few banks.
+    const int shift = (a.E >= 8 && (a.E & (a.E - 1)) == 0) ? __builtin_ctz(a.E) : 0;
+    const int stride = a.E + (shift > 0);
     int cv[kCntPerThread];
     if (a.base == nullptr) {
 #pragma unroll
@@ -429,7 +584,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
 #pragma unroll
         for (int j = 0; j < kCntPerThread; ++j) {
             const int i = threadIdx.x + 64 * kPermuteWaves * j;
-            if (i < n) s_base[i] = cv[j];
+            if (i < n) s_base[shift > 0 ? i + (i >> shift) : i] = cv[j];
         }
         __syncthreads();
         // One wave per expert column, 64 chunks per step.
@@ -437,10 +592,10 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
             int run = 0;
             for (int c0 = 0; c0 < a.nchunks; c0 += 64) {
                 const int c = c0 + lane;
-                const int val = (c < a.nchunks) ? s_base[c * a.E + e] : 0;
-                const int x = wave_inclusive_scan(val, lane);
-                if (c < a.nchunks) s_base[c * a.E + e] = run + x - val;
-                run += __shfl(x, 63);
+                const int val = (c < a.nchunks) ? s_base[c * stride + e] : 0;
+                const int x = wave_inclusive_scan(val);
+                if (c < a.nchunks) s_base[c * stride + e] = run + x - val;
+                run += __builtin_amdgcn_readlane(x, 63);
             }
             if (lane == 0) s_off[e] = run;
         }
@@ -455,7 +610,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
         for (int e0 = 0; e0 < a.E; e0 += 64) {
             const int e = e0 + lane;
             const int val = (e < a.E) ? s_off[e] : 0;
-            const int x = wave_inclusive_scan(val, lane);
+            const int x = wave_inclusive_scan(val);
             if (e < a.E) {
                 s_off[e] = run + x - val;
                 if (blockIdx.x == 0) {
@@ -463,7 +618,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
                     a.offsets[e] = run + x - val;
                 }
             }
-            run += __shfl(x, 63);
+            run += __builtin_amdgcn_readlane(x, 63);
         }
         if (blockIdx.x == 0 && lane == 0) a.offsets[a.E] = run;
     }
@@ -479,7 +634,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
         int row = -1;
         if (e >= 0 && e < a.E && rk >= 0) {
             const size_t ce = static_cast<size_t>(c) * a.E + e;
-            row = s_off[e] + (a.base != nullptr ? a.base[ce] : s_base[ce]) + rk;
+            row = s_off[e] + (a.base != nullptr ? a.base[ce] : s_base[c * stride + e]) + rk;
         }
         rows[k] = row;
         if (lane == 0) {
@@ -504,7 +659,12 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
 #pragma unroll
                 for (int u = 0; u < kCopyBatch; ++u) {
                     const int i = i0 + 64 * u + lane;
-                    if (i < nv) __builtin_nontemporal_store(v[u], dst + i);
+                    if (i >= nv) continue;
+                    if constexpr (NT) {
+                        __builtin_nontemporal_store(v[u], dst + i);
+                    } else {
+                        dst[i] = v[u];
+                    }
                 }
             }
         }
@@ -537,8 +697,12 @@ hipError_t by_k(int K, Args&&... args) {
 template <int K>
 struct RouteLaunch {
     static hipError_t run(const RouteArgs& a, hipStream_t s) {
-        if (a.E <= 8) return launch(moe_route_kernel<K, 8>, dim3((a.T + 255) / 256), dim3(256), 0, s, a);
-        return launch(moe_route_kernel<K, 16>, dim3((a.T + 255) / 256), dim3(256), 0, s, a);
+        const dim3 grid((a.T + 255) / 256), block(256);
+        if (a.E <= 8) return launch(moe_route_kernel<K, 8>, grid, block, 0, s, a);
+        if (a.E <= 16) return launch(moe_route_kernel<K, 16>, grid, block, 0, s, a);
+        const dim3 wide(static_cast<unsigned>((static_cast<long long>(a.T) + 15) / 16));
+        if (a.E <= 64) return launch(moe_route_wide_kernel<K, 4>, wide, block, 0, s, a);
+        return launch(moe_route_wide_kernel<K, 16>, wide, block, 0, s, a);
     }
 };
 
@@ -547,7 +711,9 @@ struct RankLaunch {
     static hipError_t run(const RankArgs& a, hipStream_t s) {
         const int grid = (a.nchunks + kRankWaves - 1) / kRankWaves;
         if (a.E <= 8) return launch(moe_rank_kernel<K, 8>, dim3(grid), dim3(64 * kRankWaves), 0, s, a);
-        return launch(moe_rank_kernel<K, 16>, dim3(grid), dim3(64 * kRankWaves), 0, s, a);
+        if (a.E <= kRankUnrolled) return launch(moe_rank_kernel<K, 16>, dim3(grid), dim3(64 * kRankWaves), 0, s, a);
+        if (a.E <= 64) return launch(moe_rank_wide_kernel<K, 4>, dim3(a.nchunks), dim3(kWideThreads), 0, s, a);
+        return launch(moe_rank_wide_kernel<K, 16>, dim3(a.nchunks), dim3(kWideThreads), 0, s, a);
     }
 };
 
@@ -557,10 +723,12 @@ struct PermuteLaunch {
         // One wave per token; at least one workgroup so counts and offsets
         // are written when there are no tokens.
         const int grid = a.T > 0 ? (a.T + kPermuteWaves - 1) / kPermuteWaves : 1;
-        if (a.xp != nullptr && a.vec) {
-            return launch(moe_permute_kernel<K, true>, dim3(grid), dim3(64 * kPermuteWaves), 0, s, a);
+        const dim3 block(64 * kPermuteWaves);
+        if (a.xp == nullptr || !a.vec) return launch(moe_permute_kernel<K, false, true>, dim3(grid), block, 0, s, a);
+        if (static_cast<size_t>(a.T) * K * a.hidden * sizeof(uint16_t) <= kNontemporalRows) {
+            return launch(moe_permute_kernel<K, true, true>, dim3(grid), block, 0, s, a);
         }
-        return launch(moe_permute_kernel<K, false>, dim3(grid), dim3(64 * kPermuteWaves), 0, s, a);
+        return launch(moe_permute_kernel<K, true, false>, dim3(grid), block, 0, s, a);
     }
 };
 

@@ -147,14 +147,9 @@ __global__ __launch_bounds__(kThreads) void moe_expert_gemm_kernel(const GemmArg
             const int e = e0 + lane;
             int v = 0;
             if (e < a.E) v = main_row_tiles(max(a.offsets[e + 1] - a.offsets[e], 0));
-            int x = v;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int y = __shfl_up(x, d);
-                if (lane >= d) x += y;
-            }
+            const int x = wave_inclusive_scan(v);
             if (e < a.E) s_tile0[e] = run + x - v;
-            run += __shfl(x, 63);
+            run += __builtin_amdgcn_readlane(x, 63);
         }
         if (lane == 0) s_tile0[a.E] = run;
     }

@@ -152,3 +152,51 @@ def test_dispatch_zero_tokens(dev):
     synchronize()
     assert bufs.counts.numpy().tolist() == [0] * E
     assert bufs.offsets.numpy().tolist() == [0] * (E + 1)
+
+
+def _select(row, K):
+    """K passes over a row in index order: the first untaken expert, unless a
+    later one is strictly larger (so NaN never replaces and is never replaced)."""
+    got = []
+    for _ in range(K):
+        best = None
+        for e, x in enumerate(row):
+            if e not in got and (best is None or x > row[best]):
+                best = e
+        got.append(best)
+    return got
+
+
+@pytest.mark.parametrize("T,E,K", [
+    (1, 17, 1), (63, 17, 8), (65, 33, 3), (200, 64, 8), (129, 65, 6), (70, 255, 8), (64, 256, 2),
+    (1100, 256, 4),                # 18 chunks x 256 experts: the scan kernel
+])
+def test_wide_routing_order(dev, T, E, K):
+    """More than 16 experts: ties, signed zeros, -inf and +inf rows and NaN
+    pick the experts that K passes over the row in order would."""
+    rng = np.random.default_rng(T + E)
+    logits = np.round(rng.standard_normal((T, E)) * 3).astype(np.float32)   # many ties
+    logits[0] = -np.inf
+    for r in range(1, min(T, 6)):
+        logits[r, rng.integers(0, E, size=E // 2)] = [0.0, -0.0, -np.inf, np.inf, np.nan][r - 1]
+    if T > 5:
+        logits[5, 0] = np.nan
+    x = rng.standard_normal((T, 64)).astype(np.float16)
+    want = np.array([_select(row, K) for row in logits], np.int32)
+    ids, _ = _route(logits, K)
+    assert np.array_equal(ids, want)
+    ids, w, bufs = _route_dispatch(logits, x, K)
+    assert np.array_equal(ids, want)
+    _check_dispatch(want, x, E, bufs)
+    finite = np.isfinite(logits).all(axis=1)
+    assert np.abs(w[finite] - oracle.moe_route(logits[finite], K)[1]).max(initial=0.0) <= 1e-6
+
+
+@pytest.mark.parametrize("T,E,K", [(130, 64, 8), (65, 200, 3)])
+def test_wide_dispatch_repeated_and_dropped_ids(dev, T, E, K):
+    """Caller-given ids may repeat inside a token and lie outside [0, E)."""
+    rng = np.random.default_rng(E)
+    ids = rng.integers(-2, E + 2, size=(T, K)).astype(np.int32)
+    ids[::3, 1] = ids[::3, 0]
+    x = rng.standard_normal((T, 72)).astype(np.float16)
+    _check_dispatch(ids, x, E, _dispatch(ids, x, E))
