@@ -105,19 +105,21 @@ void launch_reshape_and_cache(void* key, void* value, void* key_cache,
  * partition and keeps (max logit, exp sum, partial output) in `workspace`;
  * a second kernel rescales and reduces the partitions of every sequence
  * that has more than one (a sequence with a single partition is written by
- * the first kernel directly). For partitions of up to 1024 tokens and at
- * most a quarter as many sequences as the grid has teams of waves, the
- * first kernel runs as partition streams: every team of waves takes an
- * equal range of the batch's blocks and leaves a partial at each partition
- * end it meets; the workspace then also holds one boundary slot per wave of
- * the grid, which is sized from the current device's compute units (as is
- * the size query's answer).
- * partition_size 0 selects balanced scheduling instead: the blocks of all
- * sequences are split into equal ranges, one per team of waves, so a ragged
- * batch has no long tail; ranges that cut a sequence leave fragments that a
- * second kernel combines. Shapes it cannot take (more than 4096 sequences,
- * or teams so wide that fewer than four fit in the resident grid) fall back
- * to partitions of 512 tokens; the workspace size query covers both.
+ * the first kernel directly). partition_size is the finest cut of a large
+ * batch: an item may take several neighbouring partitions, as many as the
+ * batch's lengths leave each workgroup of the GPU. Batches of few sequences
+ * (at most two per team of workgroups, where the workspace has the room) are
+ * cut into equal ranges of blocks instead, one per team, whatever the
+ * partitions, and tables too short for a split to pay are attended in a
+ * single pass; the size query's answer depends on the current device's
+ * compute units.
+ * partition_size 0 selects balanced scheduling: the blocks of all sequences
+ * are always split into equal ranges, one per team of waves for large
+ * batches, so a ragged batch has no long tail; ranges that cut a sequence
+ * leave fragments that a second kernel combines. Shapes it cannot take (more
+ * than 4096 sequences, or teams so wide that fewer than four fit in the
+ * resident grid) fall back to partitions of 512 tokens; the workspace size
+ * query covers both.
  * `workspace` holds at least
  * swiftllm_hip_paged_attention_v2_workspace_size() bytes, 256-byte aligned;
  * it is plain scratch (no initialisation, contents unspecified after the

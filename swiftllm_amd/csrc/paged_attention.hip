@@ -66,12 +66,8 @@ struct DecodeArgs {
     int part_blocks;  // blocks per partition; 0: single pass
     int MP;           // partitions per sequence in the workspace
     int S;            // sequences
+    float share;      // split-K items: kItemShare of a resident workgroup, per block of the batch
     int snake;        // > 0: single-pass item order in snake rounds of this many
-    // Partition streams (paged_partition_stream_kernel) only:
-    float* frag;      // [W][kFragHead + gstride * D]: the piece a wave's range starts with
-    int* meta;        // [0] blocks per team q, [1] teams, [2 .. S + 2] block prefix
-    int W;            // waves in the grid
-    int stage_off;    // ints of dynamic LDS before the waves' partial slots
 };
 
 // Attends `count` blocks of one sequence: logical blocks first,
@@ -156,10 +152,51 @@ __host__ __device__ constexpr int merge_lds_floats(int G) {
     return NW * 32 + NW * (G < 16 ? G : 16) * D;
 }
 
+// Merges the NW waves' running states of one item through LDS and hands every
+// normalised output to emit(g, d, o, M, den): query head g of the gn served
+// here, dimension d, with the merged max and sum. l_run: the wave's sum over
+// its four lane groups.
+template <int D, int NW, typename Emit>
+__device__ __forceinline__ void merge_waves(float* smem, const WaveState<D>& st, float l_run, int gn,
+                                            int gstride, int w, int r, int kg, Emit emit) {
+    float* sm_m = smem;            // [NW][16]
+    float* sm_l = smem + NW * 16;  // [NW][16]
+    float* sm_o = smem + NW * 32;  // [NW][gstride][D]
+    if (kg == 0) {
+        sm_m[w * 16 + r] = st.m;
+        sm_l[w * 16 + r] = l_run;
+    }
+    if (r < gn) {
+#pragma unroll
+        for (int J = 0; J < D / 16; ++J) {
+            *reinterpret_cast<f4*>(sm_o + static_cast<size_t>(w * gstride + r) * D + 16 * J + 4 * kg) = st.acc[J];
+        }
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < gn * D; idx += NW * 64) {
+        const int g = idx / D;
+        const int d = idx - g * D;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w2 = 0; w2 < NW; ++w2) M = fmaxf(M, sm_m[w2 * 16 + g]);
+        float num = 0.0f, den = 0.0f;
+#pragma unroll
+        for (int w2 = 0; w2 < NW; ++w2) {
+            const float mw = sm_m[w2 * 16 + g];
+            const float f = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
+            num += f * sm_o[static_cast<size_t>(w2 * gstride + g) * D + d];
+            den += f * sm_l[w2 * 16 + g];
+        }
+        emit(g, d, (den > 0.0f) ? num / den : 0.0f, M, den);
+    }
+}
+
 // Bytes of the partition kernel's item list for S sequences (int prefix of
-// S + 1 entries, 16-bit sequence list of S), rounded to 16.
+// S + 1 entries, 17 int counts per group of 64 sequences, 16-bit sequence list
+// of S), rounded to 16.
 __host__ __device__ constexpr size_t part_list_lds_bytes(int S) {
-    return ((static_cast<size_t>(S) + 1) * 4 + static_cast<size_t>(S) * 2 + 15) / 16 * 16;
+    return ((static_cast<size_t>(S) + 1) * 4 + (static_cast<size_t>(S) + 63) / 64 * 17 * 4 +
+            static_cast<size_t>(S) * 2 + 15) / 16 * 16;
 }
 
 // One (sequence, kv head, head chunk, partition) item. The NW waves of the
@@ -168,7 +205,7 @@ __host__ __device__ constexpr size_t part_list_lds_bytes(int S) {
 // split-K partial. Every thread of the workgroup calls it with the same item.
 template <int D, int NW>
 __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh, int hc,
-                                            int part) {
+                                            int part, int part_blocks) {
     constexpr int NJ = D / 16;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -185,10 +222,10 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh,
     const int nblk = min((L + kBlockTokens - 1) / kBlockTokens, a.MB);
     L = min(L, nblk * kBlockTokens);
     int nparts, jb0, jb1;
-    if (a.part_blocks > 0) {
-        nparts = (nblk + a.part_blocks - 1) / a.part_blocks;
-        jb0 = part * a.part_blocks;
-        jb1 = min(nblk, jb0 + a.part_blocks);
+    if (part_blocks > 0) {
+        nparts = (nblk + part_blocks - 1) / part_blocks;
+        jb0 = part * part_blocks;
+        jb1 = min(nblk, jb0 + part_blocks);
     } else {
         nparts = 1;
         jb0 = 0;
@@ -234,47 +271,12 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh,
     const int nbw = (jb1 > first) ? (jb1 - first + NW - 1) / NW : 0;
     attend_blocks<D>(st, btrow, first, NW, nbw, L, a.kc, a.vc, a.Hkv, a.num_blocks, kvh, loff, kg,
                      qB, ident, a.scale_log2);
-    float m_run = st.m;
-    float l_run = st.l;
-    f4 (&acc)[NJ] = st.acc;
     // Per-lane partial sums cover tokens 4kg..4kg+3 of every block.
-    l_run = sum_over_kg(l_run);
-
-    // Merge the waves of this workgroup.
+    const float l_run = sum_over_kg(st.l);
     extern __shared__ __align__(16) float smem[];
-    float* sm_m = smem;            // [NW][16]
-    float* sm_l = smem + NW * 16;  // [NW][16]
-    float* sm_o = smem + NW * 32;  // [NW][gstride][D]
-    if (kg == 0) {
-        sm_m[w * 16 + r] = m_run;
-        sm_l[w * 16 + r] = l_run;
-    }
-    if (r < gn) {
-#pragma unroll
-        for (int J = 0; J < NJ; ++J) {
-            *reinterpret_cast<f4*>(sm_o + static_cast<size_t>(w * gstride + r) * D + 16 * J + 4 * kg) = acc[J];
-        }
-    }
-    __syncthreads();
-
-    const bool direct = (nparts == 1);
-    for (int idx = threadIdx.x; idx < gn * D; idx += NW * 64) {
-        const int g = idx / D;
-        const int d = idx - g * D;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w2 = 0; w2 < NW; ++w2) M = fmaxf(M, sm_m[w2 * 16 + g]);
-        float num = 0.0f, den = 0.0f;
-#pragma unroll
-        for (int w2 = 0; w2 < NW; ++w2) {
-            const float mw = sm_m[w2 * 16 + g];
-            const float f = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
-            num += f * sm_o[static_cast<size_t>(w2 * gstride + g) * D + d];
-            den += f * sm_l[w2 * 16 + g];
-        }
+    merge_waves<D, NW>(smem, st, l_run, gn, gstride, w, r, kg, [&](int g, int d, float o, float M, float den) {
         const int h = h0 + g;
-        const float o = (den > 0.0f) ? num / den : 0.0f;
-        if (direct) {
+        if (nparts == 1) {
             a.out[(static_cast<size_t>(s) * a.H + h) * D + d] = static_cast<f16>(o);
         } else {
             const size_t pi = (static_cast<size_t>(s) * a.H + h) * a.MP + part;
@@ -284,9 +286,8 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh,
                 a.ws_sum[pi] = den;
             }
         }
-    }
+    });
 }
-
 
 // At least two waves per SIMD: caps the registers (at 157 VGPRs for D=128 the
 // kernel fits three waves per SIMD), so several workgroups share a CU.
@@ -316,7 +317,7 @@ void paged_decode_kernel(const DecodeArgs a) {
         hc = blockIdx.y - kvh * a.nhc;
         s = blockIdx.z;
     }
-    decode_item<D, NW>(a, s, kvh, hc, 0);
+    decode_item<D, NW>(a, s, kvh, hc, 0, 0);
 }
 
 // Split-K partitions. The items are the real (sequence, partition) pairs
@@ -325,21 +326,49 @@ void paged_decode_kernel(const DecodeArgs a) {
 // resident workgroups, not to the worst case of every sequence, so a ragged
 // batch launches no empty workgroups (a grid over max_num_blocks_per_seq
 // would be mostly empty). Workgroups start in blockIdx order, so the order of
-// the list is the order the items start in: first every full partition
-// (part_blocks blocks), then the last, partial partition of each sequence in
+// the list is the order the items start in: first every full partition (of
+// item_blocks() blocks), then the last, partial partition of each sequence in
 // kLptClasses length classes, longest first (an empty sequence's item, which
-// writes zeros, is a partial of length 0). Measured with the gather kernel
+// writes zeros, is a partial of length 0). A single-pass call with many
+// sequences takes the same list with one partition per sequence. Measured with the gather kernel
 // of libswiftllm_ceilings on config 4's items at 1024-token partitions:
 // 151 us longest first against 166 us in sequence order.
 //
 // The item of one list position is run by several workgroups (one per kv-head
 // chunk), each with its own copy of the list, so the list must come out the
 // same in every workgroup: within a class the partials keep sequence order,
-// placed by prefix sums, never by the order atomics happen to land in.
+// placed by prefix sums, never by the order atomics happen to land in. The
+// list costs every workgroup a prologue, so it is built with one wave per
+// group of 64 sequences, class counts and ranks by ballots and sums by DPP,
+// three barriers in all; with a shuffle scan of packed class counts per chunk
+// of 256 sequences, 256 contexts of 16-128 tokens took 31.8 us instead of 27.9,
+// lognormal ones up to 8192 tokens 181.9 instead of 175.9.
 // Batches of more than kPartMaxSeqs sequences take one item per workgroup
 // over the full grid.
 constexpr int kPartMaxSeqs = 4096;
-constexpr int kLptClasses = 16;  // counted in 16-bit fields, two per int
+constexpr int kLptClasses = 16;
+
+// Blocks per item of this batch: as many whole partitions as fit in kItemShare
+// times a resident workgroup's share of all blocks, at least one. Short items
+// pay a start-up and a merge each, long ones leave a tail; longest first, an
+// item of about one share starts early enough. Measured at 512-token
+// partitions (us per call, 256 lognormal contexts up to 8192 tokens, 32/8
+// heads x 128): one partition per item 197, items of half a share 190, of one
+// 183.6, of one and a half 181.9, of two 181.7 (150 contexts of 64/8 heads:
+// 146, 133, 130, 129; 256 of 1000-4000 tokens: 406, 396, 398, 402). Every
+// workgroup of the partition kernel and every wave of its reduce works it out
+// for itself, from the lengths alone.
+constexpr float kItemShare = 1.5f;
+
+__device__ __forceinline__ int item_blocks(const int* ctx, int S, int MB, int part_blocks, float share) {
+    int sum = 0;
+    for (int i = threadIdx.x & 63; i < S; i += 64) {
+        // (2^18 blocks are 4M tokens: kPartMaxSeqs such contexts fit in an int)
+        sum += min(min((max(ctx[i], 0) + kBlockTokens - 1) / kBlockTokens, MB), 1 << 18);
+    }
+    const int most = static_cast<int>(fminf(static_cast<float>(wave_total(sum)) * share, 0x1p28f));
+    return __builtin_amdgcn_readfirstlane(part_blocks * max(1, most / part_blocks));
+}
 
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(3)))
@@ -350,133 +379,95 @@ void paged_partition_kernel(const DecodeArgs a) {
         const int part = it % a.MP;
         const int sub = (it / a.MP) % HC;
         const int s = it / (a.MP * HC);
-        if (s < a.S) decode_item<D, NW>(a, s, sub / a.nhc, sub % a.nhc, part);
+        if (s < a.S) decode_item<D, NW>(a, s, sub / a.nhc, sub % a.nhc, part, a.part_blocks);
         return;
     }
-    constexpr int kPacked = kLptClasses / 2;
-    // The item list sits in dynamic LDS after decode_item's merge area,
-    // sized by the host for this batch (part_list_lds_bytes): s_pre[S + 1]
-    // exclusive prefix of full partitions, s_part[S] sequences with a
+    // The item list sits in dynamic LDS after decode_item's merge area, sized
+    // by the host for this batch (part_list_lds_bytes): s_pre[S + 1] exclusive
+    // prefix of full partitions, s_cnt[groups of 64][kLptClasses + 1] partials
+    // per class and full partitions of each group, s_part[S] sequences with a
     // partial partition, longest first.
     extern __shared__ __align__(16) float smem[];
+    constexpr int kCols = kLptClasses + 1;
+    const int ngroups = (a.S + 63) / 64;
     int* s_pre = reinterpret_cast<int*>(smem + merge_lds_floats<D, NW>(a.G));
-    unsigned short* s_part = reinterpret_cast<unsigned short*>(s_pre + a.S + 1);
-    __shared__ int s_wpk[NW][kPacked];               // per-wave class counts of a chunk
-    __shared__ int s_cls[kLptClasses];               // next list position of each class
-    __shared__ int s_wave[NW];
+    int* s_cnt = s_pre + a.S + 1;
+    unsigned short* s_part = reinterpret_cast<unsigned short*>(s_cnt + ngroups * kCols);
+    __shared__ int s_total[2];  // full partitions, partial ones
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int pb = a.part_blocks;
-    auto nblk_of = [&](int sq) {
-        const int L = max(a.ctx[sq], 0);
-        return min((L + kBlockTokens - 1) / kBlockTokens, a.MB);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int pb = item_blocks(a.ctx, a.S, a.MB, a.part_blocks, a.share);
+    // Blocks of sequence 64 * group + lane, -1 past the batch.
+    auto nblk_of = [&](int group) {
+        const int sq = 64 * group + lane;
+        return sq < a.S ? min((max(a.ctx[sq], 0) + kBlockTokens - 1) / kBlockTokens, a.MB) : -1;
     };
     // Class of a sequence's partial partition (0 = longest), or -1 when its
     // last partition is full.
     auto class_of = [&](int nblk) {
         const int rem = nblk - (nblk / pb) * pb;
-        if (rem == 0 && nblk > 0) return -1;
-        return kLptClasses - 1 - static_cast<int>((static_cast<long long>(rem) * kLptClasses) / pb);
+        if (nblk < 0 || (rem == 0 && nblk > 0)) return -1;
+        // rem < pb <= 2^28
+        return kLptClasses - 1 - static_cast<int>(static_cast<unsigned>(rem) * kLptClasses / static_cast<unsigned>(pb));
     };
-    // Inclusive scan over the wave of 8 packed ints (two 16-bit class counts
-    // each; a workgroup chunk holds at most 256 of any class).
-    auto wave_scan8 = [&](int (&x)[kPacked]) {
+    // Counts per group of 64 sequences, one wave per group: lane k gets class
+    // k's from a ballot.
+    for (int gr = w; gr < ngroups; gr += NW) {
+        const int nblk = nblk_of(gr);
+        const int c = class_of(nblk);
+        const int full = wave_total(max(nblk, 0) / pb);
+        int n = full;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-#pragma unroll
-            for (int i = 0; i < kPacked; ++i) {
-                const int y = __shfl_up(x[i], d);
-                if (lane >= d) x[i] += y;
+        for (int k = 0; k < kLptClasses; ++k) {
+            const int nk = __popcll(__ballot(c == k));
+            if (lane == k) n = nk;
+        }
+        if (lane < kCols) s_cnt[gr * kCols + lane] = n;
+    }
+    __syncthreads();
+    // Exclusive prefixes down the groups, then the classes' first positions
+    // on top (lane k: class k; lane kLptClasses: full partitions).
+    if (w == 0) {
+        int run = 0;
+        if (lane < kCols) {
+            for (int gr = 0; gr < ngroups; ++gr) {
+                const int n = s_cnt[gr * kCols + lane];
+                s_cnt[gr * kCols + lane] = run;
+                run += n;
             }
         }
-    };
-    auto field = [](const int (&x)[kPacked], int c) { return (x[c >> 1] >> (16 * (c & 1))) & 0xffff; };
-    // Pass 1: full partitions per sequence (exclusive prefix, in chunks of
-    // the workgroup) and partials per class.
-    int carry = 0;
-    int cls_total[kPacked] = {};
-    for (int c0 = 0; c0 < a.S; c0 += NW * 64) {
-        const int sq = c0 + static_cast<int>(threadIdx.x);
-        int v = 0;
-        int pk[kPacked] = {};
-        if (sq < a.S) {
-            const int nblk = nblk_of(sq);
-            v = nblk / pb;
-            const int c = class_of(nblk);
-            if (c >= 0) pk[c >> 1] = 1 << (16 * (c & 1));
+        const int mine = lane < kLptClasses ? run : 0;
+        const int incl = wave_inclusive_scan(mine);
+        if (lane < kLptClasses) {
+            for (int gr = 0; gr < ngroups; ++gr) s_cnt[gr * kCols + lane] += incl - mine;
         }
-        int x = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int y = __shfl_up(x, d);
-            if (lane >= d) x += y;
-        }
-        wave_scan8(pk);
-        if (lane == 63) {
-            s_wave[w] = x;
-#pragma unroll
-            for (int i = 0; i < kPacked; ++i) s_wpk[w][i] = pk[i];
-        }
-        __syncthreads();
-        int before = carry, chunk = 0;
-        for (int i = 0; i < NW; ++i) {
-            before += (i < w) ? s_wave[i] : 0;
-            chunk += s_wave[i];
-#pragma unroll
-            for (int j = 0; j < kPacked; ++j) cls_total[j] += s_wpk[i][j];
-        }
-        if (sq < a.S) s_pre[sq] = before + x - v;
-        carry += chunk;
-        __syncthreads();
+        if (lane == kLptClasses) s_total[0] = run;
+        if (lane == 63) s_total[1] = incl;
     }
-    // First list position of each class (every thread holds the totals).
-    if (threadIdx.x == 0) {
-        int pos = 0;
-        for (int c = 0; c < kLptClasses; ++c) {
-            s_cls[c] = pos;
-            pos += field(cls_total, c);
-        }
-        s_pre[a.S] = carry;
-    }
-    int npartial = 0;
-#pragma unroll
-    for (int c = 0; c < kLptClasses; ++c) npartial += field(cls_total, c);
     __syncthreads();
-    // Pass 2: each partial at its class's next position, in sequence order:
-    // the position is the class cursor plus the number of lower-numbered
-    // sequences of the same class in this chunk.
-    for (int c0 = 0; c0 < a.S; c0 += NW * 64) {
-        const int sq = c0 + static_cast<int>(threadIdx.x);
-        int c = -1;
-        int pk[kPacked] = {};
-        if (sq < a.S) {
-            c = class_of(nblk_of(sq));
-            if (c >= 0) pk[c >> 1] = 1 << (16 * (c & 1));
-        }
-        int incl[kPacked];
+    // Places each sequence: its full partitions' prefix, and its partial
+    // partition at its class's next position, in sequence order.
+    for (int gr = w; gr < ngroups; gr += NW) {
+        const int nblk = nblk_of(gr);
+        const int c = class_of(nblk);
+        const int v = max(nblk, 0) / pb;
+        const int x = wave_inclusive_scan(v);
+        if (nblk >= 0) s_pre[64 * gr + lane] = s_cnt[gr * kCols + kLptClasses] + x - v;
+        unsigned long long same = 0;
 #pragma unroll
-        for (int i = 0; i < kPacked; ++i) incl[i] = pk[i];
-        wave_scan8(incl);
-        if (lane == 63) {
-#pragma unroll
-            for (int i = 0; i < kPacked; ++i) s_wpk[w][i] = incl[i];
+        for (int k = 0; k < kLptClasses; ++k) {
+            const unsigned long long m = __ballot(c == k);
+            if (c == k) same = m;
         }
-        __syncthreads();
         if (c >= 0) {
-            int rank = field(incl, c) - 1;
-            for (int i = 0; i < w; ++i) rank += (s_wpk[i][c >> 1] >> (16 * (c & 1))) & 0xffff;
-            s_part[s_cls[c] + rank] = static_cast<unsigned short>(sq);
+            const int rank = __popcll(same & ((1ull << lane) - 1ull));
+            s_part[s_cnt[gr * kCols + c] + rank] = static_cast<unsigned short>(64 * gr + lane);
         }
-        __syncthreads();
-        if (threadIdx.x < kLptClasses) {
-            int n = 0;
-            for (int i = 0; i < NW; ++i) n += (s_wpk[i][threadIdx.x >> 1] >> (16 * (threadIdx.x & 1))) & 0xffff;
-            s_cls[threadIdx.x] += n;
-        }
-        __syncthreads();
     }
-    const int nfull = carry;
-    const int total = (nfull + npartial) * HC;
+    if (threadIdx.x == 0) s_pre[a.S] = s_total[0];
+    __syncthreads();
+    const int nfull = __builtin_amdgcn_readfirstlane(s_total[0]);
+    const int total = (nfull + __builtin_amdgcn_readfirstlane(s_total[1])) * HC;
     for (int it = blockIdx.x; it < total; it += gridDim.x) {
         const int pidx = it / HC;
         const int sub = it - pidx * HC;
@@ -493,7 +484,7 @@ void paged_partition_kernel(const DecodeArgs a) {
             sq = s_part[pidx - nfull];
             part = s_pre[sq + 1] - s_pre[sq];  // after the full ones
         }
-        decode_item<D, NW>(a, sq, sub / a.nhc, sub % a.nhc, part);
+        decode_item<D, NW>(a, sq, sub / a.nhc, sub % a.nhc, part, pb);
         __syncthreads();  // the item's LDS is free again
     }
 }
@@ -667,10 +658,12 @@ struct ReduceArgs {
     const float* ws_max;
     const float* ws_sum;
     const float* ws_out;
+    int S;
     int H;
     int MB;
     int part_blocks;
     int MP;
+    float share;
 };
 
 // Combine of head h of sequence s; CH: fragment rows per load batch of the
@@ -679,7 +672,9 @@ template <int D, int CH>
 __device__ __forceinline__ void reduce_head(const ReduceArgs& a, int s, int h) {
     const int L = max(a.ctx[s], 0);
     const int nblk = min((L + kBlockTokens - 1) / kBlockTokens, a.MB);
-    const int nparts = (nblk + a.part_blocks - 1) / a.part_blocks;
+    if (nblk <= a.part_blocks) return;
+    const int pb = a.S <= kPartMaxSeqs ? item_blocks(a.ctx, a.S, a.MB, a.part_blocks, a.share) : a.part_blocks;
+    const int nparts = (nblk + pb - 1) / pb;
     if (nparts <= 1) return;
     const size_t row = static_cast<size_t>(s) * a.H + h;
     const float* pm = a.ws_max + row * a.MP;
@@ -779,12 +774,7 @@ __device__ __forceinline__ void stream_prefix(const A& a, int* s_pre, int* s_len
             v[i] = idx < n ? s_tot[idx] : 0;
             sum += v[i];
         }
-        int incl = sum;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off);
-            if (static_cast<int>(threadIdx.x) >= off) incl += t;
-        }
+        const int incl = wave_inclusive_scan(sum);
         int ex = incl - sum;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -972,163 +962,64 @@ __global__ __launch_bounds__(256) void paged_streamk_reduce_kernel(const StreamR
 }
 
 // ---------------------------------------------------------------------------
-// Split-K in partition streams. The blocks of all sequences form one list,
-// sequence by sequence, as in the balanced mode; a team of TS = Hkv * nhc
-// consecutive waves takes blocks [t*q, (t+1)*q) of it, each wave one kv head
-// and head chunk, so every wave gets the same number of blocks whatever the
-// context lengths. A wave walks its range with one continuous load pipeline
-// (the next block's tiles are in flight while a block is attended) and
-// leaves a partial (max, sum, normalised output) each time it reaches the
-// end of a partition: no LDS merge, no barrier and no pipeline drain per
-// partition, which is what the per-item walk pays over short partitions.
-// A range boundary t*q that falls strictly inside a partition splits it into
-// pieces. Only a wave's first piece can start at such a boundary; every
-// other piece starts at a partition start. A piece from a partition's start
-// goes to the partition's slot of the regular workspace, a piece from a
-// boundary to the boundary slot of wave (t, member) in `frag`. A sequence
-// with one partition and no boundary inside writes its output directly.
-// The partial of a piece that ends before the wave's range does is held in
-// the wave's LDS slot (one per wave) and written with the wave's last one,
-// so a wave's HBM writes come after its reads instead of among them (writes
-// landing in the read stream cost far more than their bytes).
-// paged_reduce_pstream_wave_kernel (up to 16 fragments per head, a wave per
-// head) and paged_reduce_pstream_split_kernel (more, four waves per head)
-// combine, per head, the partition slots and the boundary slots that fall
-// inside the sequence.
+// Split-K by teams, for batches of few sequences. The blocks of all sequences
+// form one list, as in the balanced mode, but a team is TS = Hkv * nhc
+// workgroups (one per kv head and head chunk) instead of waves: team t takes
+// blocks [t*q, (t+1)*q), q = ceil(blocks / teams), and the four waves of a
+// workgroup take a range's blocks round-robin and merge through LDS. Every
+// workgroup gets the same number of blocks whatever the context lengths, and
+// a head is left with one fragment per team that touches its sequence, at
+// most teams + 1 per sequence, whatever partition size the caller asks for.
+// A range that covers a whole sequence writes its output; otherwise its first
+// segment leaves a fragment in the workgroup's even slot and its last one in
+// the odd slot, and paged_team_reduce_kernel combines them.
+//
+// Bound: HBM for long contexts, for short ones the latency of two dependent
+// kernels. Measured on MI355X (us per call, 512-token partitions; before: a
+// range per wave, cut at partition ends, so a head of one sequence had 256
+// fragments): 1 sequence of 7919 tokens, 32/8 heads x 128, 25.1 -> 12.8; of
+// 32768 39.3 -> 27.3; 4000 tokens, 64/8 heads 49.0 -> 12.4; 8 x 32768 tokens,
+// 64/8 heads 170.5 -> 164.5 (16.8 MB of partials became 2 MB); 64 x
+// 512-4096 102.7 -> 97.1. Two workgroups per CU: three (168 registers) took
+// 14.8, 28.6, 14.0, 168.4 and 98.7 on those; one of eight waves 12.8, 27.3,
+// 11.7, 162.9 and 97.5, but 35.3 against 32.1 on 64 lognormal contexts of 8
+// heads x 64 and 54.6 against 50.4 on 32 of 16 x 128, where a segment is
+// short and its waves run dry.
 // ---------------------------------------------------------------------------
+constexpr int kTeamWaves = 4;
+constexpr int kTeamPerCU = 2;  // workgroups per CU: two waves per SIMD
 
-// A wave-uniform pointer held in SGPRs at this point of the program: the
-// empty asm hides its value from the optimiser, so address arithmetic on it
-// is done where it is used instead of being hoisted into a loop-invariant
-// 64-bit vector register pair.
-__device__ __forceinline__ char* pinned_sgpr(char* p) {
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
-// Attends blocks j0 .. j1 - 1 of one sequence in order, double-buffered like
-// attend_blocks, and calls done(j) after block j; the next block's loads are
-// in flight while done(j) runs.
-template <int D, typename Done>
-__device__ __forceinline__ void attend_run(WaveState<D>& st, const const_int* btrow, int j0, int j1,
-                                           int L, const f16* kc, const f16* vc, int Hkv,
-                                           int num_blocks, int kvh, int loff, int kg,
-                                           const QOperand<D>& qB, h4 ident, float scale_log2,
-                                           Done done) {
-    constexpr int NJ = D / 16;
-    const int count = j1 - j0;
-    if (count <= 0) return;
-    auto block_at = [&](int j) { return __builtin_amdgcn_readfirstlane(btrow[j]); };
-    auto valid_of = [&](int j, int b) {
-        return block_ok(b, num_blocks) ? min(kBlockTokens, L - j * kBlockTokens) : 0;
-    };
-    h4 kA[NJ], vA[NJ], kB[NJ], vB[NJ];
-    int jA = j0;
-    int bA = block_at(jA);
-    load_tile<D>(kc, vc, Hkv, num_blocks, bA, kvh, loff, kA, vA);
-    int left = count;
-    for (; left > 2; left -= 2) {
-        const int jB = jA + 1;
-        const int bB = block_at(jB);
-        load_tile<D>(kc, vc, Hkv, num_blocks, bB, kvh, loff, kB, vB);
-        attend_block<D>(st, valid_of(jA, bA), kg, kA, vA, qB, ident, scale_log2);
-        done(jA);
-        jA = jB + 1;
-        bA = block_at(jA);
-        load_tile<D>(kc, vc, Hkv, num_blocks, bA, kvh, loff, kA, vA);
-        attend_block<D>(st, valid_of(jB, bB), kg, kB, vB, qB, ident, scale_log2);
-        done(jB);
-    }
-    if (left == 2) {
-        const int jB = jA + 1;
-        const int bB = block_at(jB);
-        load_tile<D>(kc, vc, Hkv, num_blocks, bB, kvh, loff, kB, vB);
-        attend_block<D>(st, valid_of(jA, bA), kg, kA, vA, qB, ident, scale_log2);
-        done(jA);
-        attend_block<D>(st, valid_of(jB, bB), kg, kB, vB, qB, ident, scale_log2);
-        done(jB);
-    } else {
-        attend_block<D>(st, valid_of(jA, bA), kg, kA, vA, qB, ident, scale_log2);
-        done(jA);
-    }
-}
-
-// Partition streams serve partitions of up to kPStreamMaxPartBlocks blocks,
-// in batches whose block prefix fits in LDS, with a grid of
-// kPStreamWavesPerSimd waves per SIMD (the kernel's register cap).
-#ifndef SWIFTLLM_PSTREAM_MAX_PART_BLOCKS
-#define SWIFTLLM_PSTREAM_MAX_PART_BLOCKS 64
-#endif
-#ifndef SWIFTLLM_PSTREAM_WAVES_PER_SIMD
-#define SWIFTLLM_PSTREAM_WAVES_PER_SIMD 2
-#endif
-constexpr int kPStreamMaxPartBlocks = SWIFTLLM_PSTREAM_MAX_PART_BLOCKS;
-constexpr int kPStreamWavesPerSimd = SWIFTLLM_PSTREAM_WAVES_PER_SIMD;
-
-// Teams of a partition-stream grid of W waves, TS waves per team.
-__host__ __device__ __forceinline__ int pstream_teams(int W, int TS) { return max(1, W / TS); }
-
-// Where a piece's partial goes: rows (lane row r at rows + r * rstride, 16
-// bytes per lane group and 16-row slice), max and sum (row r at m / l +
-// r * mstride). Wave-uniform.
-struct PieceDst {
-    char* rows;
-    char* m;
-    char* l;
-    unsigned rstride;
-    unsigned mstride;
+struct TeamArgs {
+    f16* out;
+    const f16* q;
+    const f16* kc;
+    const f16* vc;
+    const int* bt;
+    const int* ctx;
+    float* frag;  // [2 * teams * TS][kFragHead + gstride * D]
+    int* meta;    // for the reduce: [0] blocks per team, [1 .. S + 1] block prefix
+    float scale_log2;
+    int S, H, Hkv, G, nhc, MB, num_blocks;
+    int teams;
 };
 
-// Floats a lane keeps in its LDS slot: its NJ output vectors, max and sum
-// (padded to 16 bytes).
 template <int D>
-constexpr int kStageFloats = 4 * (D / 16) + 4;
-
-// Writes a piece's partial: lane (r, kg) its four outputs of each 16-row
-// slice of row r, lanes with kg = 0 the row's max and sum; rows r >= gn
-// (padding) are skipped. The lane offsets are computed here from the lane
-// index (behind an empty asm), so none stays live in a register.
-template <int D>
-__device__ __forceinline__ void write_piece(const PieceDst& d, int lane, bool row_ok, const f4 (&v)[D / 16],
-                                            float m, float l) {
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-    const unsigned rr = static_cast<unsigned>(ln & 15);
-    const unsigned kk = static_cast<unsigned>(ln >> 4);
-    char* rows = pinned_sgpr(d.rows);
-    if (row_ok) {
-        const unsigned lo = rr * d.rstride + 16u * kk;
-#pragma unroll
-        for (int J = 0; J < D / 16; ++J) __builtin_nontemporal_store(v[J], reinterpret_cast<f4*>(rows + lo + 64u * J));
-        if (kk == 0) {
-            *reinterpret_cast<float*>(pinned_sgpr(d.m) + rr * d.mstride) = m;
-            *reinterpret_cast<float*>(pinned_sgpr(d.l) + rr * d.mstride) = l;
-        }
-    }
-}
-
-template <int D>
-__global__ __launch_bounds__(64 * kStreamWaves) __attribute__((amdgpu_waves_per_eu(kPStreamWavesPerSimd)))
-void paged_partition_stream_kernel(const DecodeArgs a) {
+__global__ __launch_bounds__(64 * kTeamWaves) __attribute__((amdgpu_waves_per_eu(kTeamPerCU)))
+void paged_team_kernel(const TeamArgs a) {
     constexpr int NJ = D / 16;
-    extern __shared__ int s_dyn[];
-    int* s_pre = s_dyn;              // [S + 1]
-    int* s_len = s_dyn + a.S + 1;    // [S]
-    __shared__ int s_tot[64 * kStreamWaves];
+    constexpr int NW = kTeamWaves;
+    extern __shared__ __align__(16) float smem[];
+    const int gstride = min(16, a.G);
+    int* s_pre = reinterpret_cast<int*>(smem + merge_lds_floats<D, NW>(a.G));  // [S + 1]
+    int* s_len = s_pre + a.S + 1;                                              // [S]
+    __shared__ int s_tot[64 * NW];
     stream_prefix(a, s_pre, s_len, s_tot);
 
     const int U = __builtin_amdgcn_readfirstlane(s_pre[a.S]);
-    const int P = a.part_blocks;
-    const int TS = a.Hkv * a.nhc;
-    const int teams = pstream_teams(a.W, TS);
-    const int q = (U + teams - 1) / teams;
+    const int q = (U + a.teams - 1) / a.teams;
     if (blockIdx.x == 0) {
-        // For the reduce: blocks per team, teams, and the block prefix.
-        for (int i = threadIdx.x; i <= a.S; i += blockDim.x) a.meta[2 + i] = s_pre[i];
-        if (threadIdx.x == 0) {
-            a.meta[0] = q;
-            a.meta[1] = teams;
-        }
+        for (int i = threadIdx.x; i <= a.S; i += blockDim.x) a.meta[1 + i] = s_pre[i];
+        if (threadIdx.x == 0) a.meta[0] = q;
     }
     // Sequences without blocks are not in the list: zero their outputs here.
     for (int sz = blockIdx.x; sz < a.S; sz += gridDim.x) {
@@ -1138,15 +1029,13 @@ void paged_partition_stream_kernel(const DecodeArgs a) {
             }
         }
     }
-
     const int lane = threadIdx.x & 63;
-    const int w = blockIdx.x * kStreamWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int team = w / TS;
-    if (team >= teams || U == 0) return;
-    const int member = w - team * TS;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15;
     const int kg = lane >> 4;
-    const int gstride = min(16, a.G);
+    const int TS = a.Hkv * a.nhc;
+    const int team = blockIdx.x / TS;
+    const int member = blockIdx.x - team * TS;
     const int kvh = member / a.nhc;
     const int hc = member - kvh * a.nhc;
     const int g0 = hc * 16;
@@ -1161,32 +1050,21 @@ void paged_partition_stream_kernel(const DecodeArgs a) {
         ident[i] = (4 * kg + i == r) ? static_cast<f16>(1.0f) : static_cast<f16>(0.0f);
     }
     const int loff = kv_elem_offset(r, 4 * kg);
-
-    // One partial per wave can wait in LDS (this wave's 64-lane slot) for the
-    // end of the wave's range.
-    float* slot = reinterpret_cast<float*>(s_dyn + a.stage_off) +
-                  (static_cast<size_t>(threadIdx.x >> 6) * 64 + lane) * kStageFloats<D>;
-    bool staged = false;
-    PieceDst held{};
-
     int u = u0;
     while (u < u1) {
-        // Sequence of block u: the largest s with s_pre[s] <= u. Wave-uniform
-        // values go through readfirstlane so the block-table reads stay
-        // scalar loads.
         int lo = 0, hi = a.S;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (s_pre[mid] <= u) lo = mid; else hi = mid;
         }
+        // Wave-uniform, in scalar registers, so the block-table reads stay
+        // scalar loads.
         const int s = __builtin_amdgcn_readfirstlane(lo);
         const int L = __builtin_amdgcn_readfirstlane(s_len[s]);
         const int pre = __builtin_amdgcn_readfirstlane(s_pre[s]);
         const int nb = __builtin_amdgcn_readfirstlane(s_pre[s + 1]) - pre;
         const int j0 = u - pre;
-        const int j1 = min(nb, u1 - pre);
-        const int nparts = (nb + P - 1) / P;
-
+        const int seg = min(nb - j0, u1 - u);
         QOperand<D> qB;
         {
             const f16* qp = a.q + (static_cast<size_t>(s) * a.H + h0 + min(r, gn - 1)) * D + 4 * kg;
@@ -1202,175 +1080,63 @@ void paged_partition_stream_kernel(const DecodeArgs a) {
         st.l = 0.0f;
 #pragma unroll
         for (int J = 0; J < NJ; ++J) st.acc[J] = f4{0, 0, 0, 0};
-        int seg0 = j0;                            // first block of the open piece
-        int cut = min(j1, (j0 / P + 1) * P);      // block after the open piece
-        attend_run<D>(st, btrow, j0, j1, L, a.kc, a.vc, a.Hkv, a.num_blocks, kvh, loff, kg, qB,
-                      ident, a.scale_log2, [&](int j) {
-            if (j + 1 != cut) return;
-            const int part = seg0 / P;
-            const float l_run = sum_over_kg(st.l);
-            const float inv = (l_run > 0.0f) ? 1.0f / l_run : 0.0f;
-            const bool whole = (seg0 == part * P) && (cut == min(nb, (part + 1) * P));
-            const size_t row0 = static_cast<size_t>(s) * a.H + h0;
-            if (whole && nparts == 1) {
-                // Lane offsets computed here from the lane index, so no lane
-                // address stays live across the block loop (the kernel runs
-                // at its 168-register cap).
-                int ln = lane;
-                asm volatile("" : "+v"(ln));
-                const int rr = ln & 15;
-                const int kk = ln >> 4;
-                char* ob = pinned_sgpr(reinterpret_cast<char*>(a.out + row0 * D));
-                const unsigned lo = static_cast<unsigned>(rr * D + 4 * kk) * sizeof(f16);
-                if (r < gn) {
-#pragma unroll
-                    for (int J = 0; J < NJ; ++J) {
-                        h4 o;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) o[i] = static_cast<f16>(st.acc[J][i] * inv);
-                        *reinterpret_cast<h4*>(ob + lo + 32u * J) = o;
-                    }
-                }
-                // The compiler treats the wave's memory counter as out of
-                // order while stores and loads are both in flight, and then
-                // waits for every load before each block: a full wait here
-                // keeps the waits in the block loop exact.
-                wait_vm<0>();
+        attend_blocks<D>(st, btrow, j0 + w, NW, (seg - w + NW - 1) / NW, L, a.kc, a.vc, a.Hkv,
+                         a.num_blocks, kvh, loff, kg, qB, ident, a.scale_log2);
+        const float l_run = sum_over_kg(st.l);
+        const bool direct = j0 == 0 && seg == nb;
+        float* f = a.frag + static_cast<size_t>(2 * blockIdx.x + (u != u0)) * (kFragHead + gstride * D);
+        if (u != u0) __syncthreads();  // the segment before has been read from LDS
+        merge_waves<D, NW>(smem, st, l_run, gn, gstride, w, r, kg, [&](int g, int d, float o, float M, float den) {
+            if (direct) {
+                a.out[(static_cast<size_t>(s) * a.H + h0 + g) * D + d] = static_cast<f16>(o);
             } else {
-                // A partition slot (the piece starts at its partition's
-                // start) or the wave's boundary slot.
-                PieceDst dst;
-                if (seg0 == part * P) {
-                    const size_t p0 = row0 * a.MP + part;
-                    dst.rows = reinterpret_cast<char*>(a.ws_out + p0 * D);
-                    dst.rstride = static_cast<unsigned>(a.MP) * D * sizeof(float);
-                    dst.m = reinterpret_cast<char*>(a.ws_max + p0);
-                    dst.l = reinterpret_cast<char*>(a.ws_sum + p0);
-                    dst.mstride = static_cast<unsigned>(a.MP) * sizeof(float);
-                } else {
-                    char* f = reinterpret_cast<char*>(a.frag + static_cast<size_t>(w) * (kFragHead + gstride * D));
-                    dst.rows = f + kFragHead * sizeof(float);
-                    dst.rstride = D * sizeof(float);
-                    dst.m = f;
-                    dst.l = f + 16 * sizeof(float);
-                    dst.mstride = sizeof(float);
-                }
-                if (!staged && pre + cut != u1) {
-                    // Held in LDS until the wave's range ends, so that its
-                    // HBM writes do not land among the wave's reads.
-#pragma unroll
-                    for (int J = 0; J < NJ; ++J) *reinterpret_cast<f4*>(slot + 4 * J) = st.acc[J] * inv;
-                    slot[4 * NJ] = st.m;
-                    slot[4 * NJ + 1] = l_run;
-                    held = dst;
-                    staged = true;
-                } else {
-                    f4 v[NJ];
-#pragma unroll
-                    for (int J = 0; J < NJ; ++J) v[J] = st.acc[J] * inv;
-                    write_piece<D>(dst, lane, r < gn, v, st.m, l_run);
-                    wait_vm<0>();
+                f[kFragHead + g * D + d] = o;
+                if (d == 0) {
+                    f[g] = M;
+                    f[16 + g] = den;
                 }
             }
-            st.m = -INFINITY;
-            st.l = 0.0f;
-#pragma unroll
-            for (int J = 0; J < NJ; ++J) st.acc[J] = f4{0, 0, 0, 0};
-            seg0 = cut;
-            cut = min(j1, cut + P);
         });
-        u = pre + j1;
-    }
-    if (staged) {
-        f4 v[NJ];
-#pragma unroll
-        for (int J = 0; J < NJ; ++J) v[J] = *reinterpret_cast<const f4*>(slot + 4 * J);
-        write_piece<D>(held, lane, r < gn, v, slot[4 * NJ], slot[4 * NJ + 1]);
+        u += seg;
     }
 }
 
-// Reduce of the partition streams: one (query head, sequence) combines its
-// nparts partition slots and the boundary slots of teams ta .. tb whose
-// boundary falls strictly inside the sequence's blocks. A boundary at a
-// partition start splits nothing; its fragment is given weight 0 (and the
-// partition slot 0 row, which is finite, as its row).
-struct PStreamReduceArgs {
+// One (query head, sequence) per workgroup: its fragments come from the teams
+// whose ranges touch the sequence. A fragment is its team's first segment
+// (even slot) unless the sequence starts inside that team's range.
+struct TeamReduceArgs {
     f16* out;
-    const float* ws_max;
-    const float* ws_sum;
-    const float* ws_out;
     const float* frag;
     const int* meta;
-    int H, G, nhc, MP, part_blocks, gstride, TS;
+    int H, G, nhc, TS, gstride;
 };
 
-// CH: fragment rows per batch of the one-wave combine; 0: the head is
-// combined by the four waves of the workgroup (combine_head_split).
-template <int D, int CH>
-__device__ __forceinline__ void pstream_reduce_head(const PStreamReduceArgs& a, int s, int h) {
+template <int D>
+__global__ __launch_bounds__(256) void paged_team_reduce_kernel(const TeamReduceArgs a) {
+    const int s = blockIdx.y;
+    const int h = blockIdx.x;
     const int q = a.meta[0];
-    const int pre = a.meta[2 + s];
-    const int nb = a.meta[3 + s] - pre;
-    const int P = a.part_blocks;
-    const int nparts = (nb + P - 1) / P;
-    // Boundaries t*q strictly inside (pre, pre + nb). When q and pre are
-    // multiples of P every boundary falls on a partition start and splits
-    // nothing, so none is combined.
-    const int ta = pre / q + 1;
-    const int tb = nb > 0 ? (pre + nb - 1) / q : ta - 1;
-    const bool on_starts = (q % P == 0) && (pre % P == 0);
-    const int nbound = on_starts ? 0 : max(0, tb - ta + 1);
-    if (nb == 0 || (nparts == 1 && nbound == 0)) return;  // zeros or written directly
+    const int pre = a.meta[1 + s];
+    const int nb = a.meta[2 + s] - pre;
+    if (nb == 0) return;
+    const int ta = pre / q;
+    const int P = (pre + nb - 1) / q - ta + 1;
+    if (P == 1) return;  // written by its team
     const int kvh = h / a.G;
     const int gk = h - kvh * a.G;
     const int hc = gk / 16;
     const int g = gk - hc * 16;
     const int member = kvh * a.nhc + hc;
-    const size_t row = static_cast<size_t>(s) * a.H + h;
-    const float* pm = a.ws_max + row * a.MP;
-    const float* pl = a.ws_sum + row * a.MP;
-    const float* po = a.ws_out + row * a.MP * D;
     const size_t fs = kFragHead + static_cast<size_t>(a.gstride) * D;
-    auto split = [&](int i) {  // boundary fragment i: a piece of its own?
-        const int t = ta + i;
-        return (t * q - pre) % P != 0;
+    const bool late = pre > ta * q;  // the sequence starts inside its first team's range
+    auto frag_of = [&](int i) {
+        return a.frag + static_cast<size_t>(2 * ((ta + i) * a.TS + member) + (i == 0 && late)) * fs;
     };
-    auto frag_of = [&](int i) { return a.frag + static_cast<size_t>((ta + i) * a.TS + member) * fs; };
-    auto fm = [&](int p) {
-        if (p < nparts) return pm[p];
-        const int i = p - nparts;
-        return split(i) ? frag_of(i)[g] : -INFINITY;
-    };
-    auto fl = [&](int p) {
-        if (p < nparts) return pl[p];
-        const int i = p - nparts;
-        return split(i) ? frag_of(i)[16 + g] : 0.0f;
-    };
-    auto fo = [&](int p) {
-        if (p < nparts) return po + static_cast<size_t>(p) * D;
-        const int i = p - nparts;
-        return split(i) ? frag_of(i) + kFragHead + static_cast<size_t>(g) * D : po;
-    };
-    f16* o = a.out + row * D;
-    auto out = [&](int d, float v) { o[d] = static_cast<f16>(v); };
-    if constexpr (CH == 0) {
-        combine_head_split<D, 4>(nparts + nbound, fm, fl, fo, out);
-    } else {
-        combine_head_wave<D, CH>(nparts + nbound, fm, fl, fo, out);
-    }
-}
-
-template <int D, int CH>
-__global__ __launch_bounds__(256) void paged_reduce_pstream_wave_kernel(const PStreamReduceArgs a) {
-    const int h = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (h >= a.H) return;
-    pstream_reduce_head<D, CH>(a, blockIdx.y, h);
-}
-
-// One (query head, sequence) per workgroup of four waves.
-template <int D>
-__global__ __launch_bounds__(256) void paged_reduce_pstream_split_kernel(const PStreamReduceArgs a) {
-    pstream_reduce_head<D, 0>(a, blockIdx.y, blockIdx.x);
+    f16* o = a.out + (static_cast<size_t>(s) * a.H + h) * D;
+    combine_head_split<D, 4>(
+        P, [&](int i) { return frag_of(i)[g]; }, [&](int i) { return frag_of(i)[16 + g]; },
+        [&](int i) { return frag_of(i) + kFragHead + static_cast<size_t>(g) * D; },
+        [&](int d, float v) { o[d] = static_cast<f16>(v); });
 }
 
 // Bit-exact materialisation of one (sequence, kv head) through the tile
@@ -1472,6 +1238,10 @@ int validate_decode(const char* who, const void* out, const void* q, const void*
 #define SWIFTLLM_WAVES_V1 4
 #endif
 constexpr int kWavesV1 = SWIFTLLM_WAVES_V1;
+constexpr int kWavesV1Wide = 8;
+// Blocks per sequence up to which several rounds of single-pass workgroups
+// run in plain order.
+constexpr int kSingleRoundBlocks = 64;
 // Waves per workgroup of a split-K partition.
 #ifndef SWIFTLLM_WAVES_V2
 #define SWIFTLLM_WAVES_V2 4
@@ -1499,6 +1269,12 @@ hipError_t launch_partition_t(const DecodeArgs& a, unsigned grid, hipStream_t st
 }
 
 int device_cus();
+
+// kItemShare of what one of the partition kernel's resident workgroups (three
+// per CU) gets of a batch, per block of it.
+float item_share(const DecodeArgs& a) {
+    return kItemShare * static_cast<float>(a.Hkv * a.nhc) / static_cast<float>(3 * device_cus());
+}
 
 // Split-K partition kernel: a grid of resident workgroups (three 4-wave
 // workgroups per CU, four rounds) walking the compacted item list, or one
@@ -1546,29 +1322,59 @@ int decode_v1(void* out, const void* q, const void* kc, const void* vc, const in
     DecodeArgs a = make_args(out, q, kc, vc, bt, ctx, scale, sh, num_blocks);
     a.part_blocks = 0;
     a.MP = 1;
-    // Snake order over the ranked sequences when the whole grid is resident
-    // at once (three 4-wave workgroups per CU at the kernel's register count)
-    // and small enough to rank; otherwise sequence order, balanced by the
-    // dispatcher as workgroups finish.
+    const int cus = device_cus();
     const long long items = static_cast<long long>(sh.S) * a.Hkv * a.nhc;
-    a.snake = (kWavesV1 == 4 && sh.S <= kLptMaxSeqs && items <= 3LL * device_cus()) ? device_cus() : 0;
+    // At most one workgroup per CU: eight waves each, so a context is half as
+    // long a chain (16 query heads would need more LDS for the merge).
+    // Measured (us per call, 4 waves -> 8): 1 x 1024 tokens of 32/8 heads x 128
+    // 12.5 -> 11.4, 32 x 512 13.9 -> 12.4, 4 x 2048 of 8 heads x 64 16.5 ->
+    // 13.7. At 64 x 32-512 (512 items) 15.8 -> 18.5, so not beyond.
+    if (items <= cus && a.G <= 8) {
+        return launched(launch_decode<kWavesV1Wide>(a, sh.D, sh.S, 1, stream), who);
+    }
+    if (items <= 3LL * cus) {
+        // The whole grid is resident at once (three 4-wave workgroups per CU
+        // at the kernel's register count): snake order over the ranked
+        // sequences when there are few enough to rank.
+        a.snake = sh.S <= kLptMaxSeqs ? cus : 0;
+    } else if (sh.MB > kSingleRoundBlocks && sh.S <= kPartMaxSeqs) {
+        // Several rounds of workgroups, and contexts long enough for the last
+        // ones to leave a tail: the item list, longest first, one item per
+        // sequence and kv head. Measured (us per call, plain order -> list):
+        // lognormal contexts, 32/8 heads x 128, 256 up to 8192 tokens 243 ->
+        // 182, up to 2048 147 -> 131, 140 up to 8192 168 -> 136; 256 of
+        // 1000-4000 413 -> 394; but 256 of 16-128 18.8 -> 28.
+        a.part_blocks = std::min(sh.MB, 1 << 27);  // 2^31 tokens
+        a.share = item_share(a);
+        bool too_large = false;
+        return launched(launch_partition<kWavesV2>(a, sh.D, stream, &too_large), who);
+    }
     return launched(launch_decode<kWavesV1>(a, sh.D, sh.S, 1, stream), who);
 }
 
-constexpr int kPStreamWavesPerCU = 4 * kPStreamWavesPerSimd;
+// Whether a split-K call runs single pass instead: its tables are too short
+// for a split to pay for the second kernel. The longest context is at most MB
+// blocks; a single pass takes about 5 us + 0.08-0.165 us per block of it, a
+// split 7.5-9.5 us at least, and with items enough for every CU the single
+// pass reads at the same rate. Measured (us per call, single pass / teams,
+// all contexts of one length, 32/8 heads x 128): 1 sequence of 512 tokens 7.8
+// / 8.2, of 1024 11.4 / 9.1; 8 of 512 9.2 / 10.8, of 1024 14.9 / 12.8; 16 of
+// 1024 16.4 / 17.4, of 2048 29.3 / 27.2; 32 of 2048 41.6 / 46.8; 64 of
+// 64-1024 25.9 / 34.1; items: 128 of 200-400 28.8 / 31.0, 256 of 1-1024
+// lognormal 106 / 105.
+bool single_pass(const Shape& sh, int cus) {
+    if (sh.S > kPartMaxSeqs) return false;
+    const long long items = static_cast<long long>(sh.S) * sh.Hkv * ((sh.H / sh.Hkv + 15) / 16);
+    return sh.MB <= (items <= 3LL * cus ? 32 + items / 4 : kSingleRoundBlocks);
+}
 
 // Split-K workspace: max logits and exp sums [S][H][MP] and partial outputs
-// [S][H][MP][D], all fp32; with partition streams also the boundary pieces
-// [W][kFragHead + gstride * D] and the team metadata (q, teams, block
-// prefix [S + 1]). Plain scratch: every value a call reads was written
-// earlier in the same call, so it needs no initialisation.
+// [S][H][MP][D], all fp32, or the teams' fragments and their metadata. Plain
+// scratch: every value a call reads was written earlier in the same call, so
+// it needs no initialisation.
 struct V2Need {
     int MP;          // partitions per sequence
     size_t stat;     // bytes of one [S][H][MP] float array
-    bool pstream;    // partition streams
-    int W;           // waves of the partition-stream grid
-    size_t frag;     // offset of the boundary pieces
-    size_t meta;     // offset of the team metadata
     size_t total;    // bytes of the whole workspace
 };
 
@@ -1578,22 +1384,45 @@ V2Need v2_need(const Shape& sh, int partition_size, int cus) {
     n.MP = sh.MB == 0 ? 1 : (sh.MB + part_blocks - 1) / part_blocks;
     n.stat = align_up(sizeof(float) * static_cast<size_t>(sh.S) * sh.H * n.MP);
     n.total = 2 * n.stat + align_up(sizeof(float) * static_cast<size_t>(sh.S) * sh.H * n.MP * sh.D);
+    // Few sequences and short partitions: room for eight fragments per CU and
+    // the block prefix beside the partials. The teams need half of it; the
+    // size is part of what callers have stored and stays.
     const int G = sh.H / sh.Hkv;
     const long long TS = static_cast<long long>(sh.Hkv) * ((G + 15) / 16);
-    n.W = cus * kPStreamWavesPerCU;
-    // Partition streams when partitions are short and the batch has at most
-    // a quarter as many sequences as the grid has teams (a wave then starts
-    // few new sequences, each a pipeline restart), and the lane offsets of
-    // a wave's partial rows fit in 31 bits.
-    const long long teams = TS > 0 ? n.W / TS : 0;
-    n.pstream = sh.S <= kStreamMaxSeqs && part_blocks <= kPStreamMaxPartBlocks && TS > 0 && TS <= n.W &&
-                4LL * sh.S <= teams && 64LL * n.MP * sh.D < (1LL << 31);
-    if (n.pstream) {
+    const long long W = 8LL * cus;
+    const long long teams = TS > 0 ? W / TS : 0;
+    if (sh.S <= kStreamMaxSeqs && part_blocks <= 64 && TS > 0 && TS <= W && 4LL * sh.S <= teams &&
+        64LL * n.MP * sh.D < (1LL << 31)) {
         const size_t gstride = static_cast<size_t>(std::min(16, G));
-        n.frag = n.total;
-        n.meta = n.frag + align_up(sizeof(float) * static_cast<size_t>(n.W) * (kFragHead + gstride * sh.D));
-        n.total = n.meta + align_up(sizeof(int) * (static_cast<size_t>(sh.S) + 3));
+        n.total += align_up(sizeof(float) * static_cast<size_t>(W) * (kFragHead + gstride * sh.D)) +
+                   align_up(sizeof(int) * (static_cast<size_t>(sh.S) + 3));
     }
+    return n;
+}
+
+// The team kernel's grid and workspace; teams == 0 where it does not serve
+// the shape: fewer than four teams, or more than two sequences per team,
+// which then have items enough for the GPU and longer ranges of their own.
+// Measured (us per call, 32/8 heads x 128, contexts lognormal around 600):
+// 100 sequences 87.6 by teams, 89.8 in items of 512-token partitions; 256
+// 191.9 by teams, 179 in items (below).
+struct TeamNeed {
+    int teams, TS;
+    size_t meta;   // offset of the metadata behind the fragments
+    size_t total;
+};
+
+TeamNeed team_need(const Shape& sh, int cus) {
+    TeamNeed n{};
+    const int G = sh.H / sh.Hkv;
+    const long long TS = static_cast<long long>(sh.Hkv) * ((G + 15) / 16);
+    const long long teams = static_cast<long long>(cus) * kTeamPerCU / TS;
+    if (teams < 4 || sh.S > 2 * teams || sh.S > kStreamMaxSeqs) return n;
+    n.teams = static_cast<int>(teams);
+    n.TS = static_cast<int>(TS);
+    n.meta = align_up(sizeof(float) * 2 * static_cast<size_t>(teams * TS) *
+                      (kFragHead + static_cast<size_t>(std::min(16, G)) * sh.D));
+    n.total = n.meta + sizeof(int) * (static_cast<size_t>(sh.S) + 2);
     return n;
 }
 
@@ -1649,14 +1478,9 @@ StreamNeed stream_need(const Shape& sh, int cus) {
     return n;
 }
 
-int decode_balanced(void* out, void* ws, size_t ws_bytes, const void* q, const void* kc,
+int decode_balanced(void* out, void* ws, const StreamNeed& need, const void* q, const void* kc,
                     const void* vc, const int* bt, const int* ctx, float scale, const Shape& sh,
                     int num_blocks, hipStream_t stream, const char* who) {
-    const StreamNeed need = stream_need(sh, device_cus());
-    if (ws_bytes < need.total) {
-        return fail(SWIFTLLM_ERR_INVALID_PARAMETER, "%s: workspace of %zu bytes, %zu needed", who,
-                    ws_bytes, need.total);
-    }
     DecodeArgs d = make_args(out, q, kc, vc, bt, ctx, scale, sh, num_blocks);
     StreamArgs a{};
     a.out = d.out;
@@ -1715,49 +1539,50 @@ size_t v2_bytes(const Shape& sh, int partition_size, int cus) {
     return partition_size == 0 ? stream_need(sh, cus).total : v2_need(sh, partition_size, cus).total;
 }
 
-// Partition streams, then their reduce (which also combines a partition
-// split by a range boundary when the sequence has one partition).
-int decode_pstream(DecodeArgs& a, char* base, const V2Need& need, const Shape& sh,
-                   hipStream_t stream, const char* who) {
-    a.frag = reinterpret_cast<float*>(base + need.frag);
-    a.meta = reinterpret_cast<int*>(base + need.meta);
-    a.W = need.W;
-    // Dynamic LDS: the block prefix and lengths (2S + 1 ints), then every
-    // wave's slot for one held partial (16-byte aligned).
-    a.stage_off = static_cast<int>((2 * static_cast<size_t>(sh.S) + 1 + 3) & ~static_cast<size_t>(3));
-    const size_t stage = static_cast<size_t>(kStreamWaves) * 64 * sizeof(float) *
-                         (sh.D == 128 ? kStageFloats<128> : kStageFloats<64>);
-    const size_t lds = sizeof(int) * static_cast<size_t>(a.stage_off) + stage;
-    const dim3 grid(need.W / kStreamWaves);
-    hipError_t err = sh.D == 128
-        ? launch(paged_partition_stream_kernel<128>, grid, dim3(64 * kStreamWaves), lds, stream, a)
-        : launch(paged_partition_stream_kernel<64>, grid, dim3(64 * kStreamWaves), lds, stream, a);
+// The team kernel, then its reduce; ws holds need.total bytes.
+int decode_team(void* out, void* ws, const void* q, const void* kc, const void* vc, const int* bt,
+                const int* ctx, float scale, const Shape& sh, int num_blocks, const TeamNeed& need,
+                hipStream_t stream, const char* who) {
+    const DecodeArgs d = make_args(out, q, kc, vc, bt, ctx, scale, sh, num_blocks);
+    TeamArgs a{};
+    a.out = d.out;
+    a.q = d.q;
+    a.kc = d.kc;
+    a.vc = d.vc;
+    a.bt = bt;
+    a.ctx = ctx;
+    a.frag = static_cast<float*>(ws);
+    a.meta = reinterpret_cast<int*>(static_cast<char*>(ws) + need.meta);
+    a.scale_log2 = d.scale_log2;
+    a.S = sh.S;
+    a.H = sh.H;
+    a.Hkv = sh.Hkv;
+    a.G = d.G;
+    a.nhc = d.nhc;
+    a.MB = sh.MB;
+    a.num_blocks = num_blocks;
+    a.teams = need.teams;
+    // Dynamic LDS: the wave merge, then the block prefix and the lengths.
+    const size_t merge = sizeof(float) * static_cast<size_t>(sh.D == 128 ? merge_lds_floats<128, kTeamWaves>(a.G)
+                                                                         : merge_lds_floats<64, kTeamWaves>(a.G));
+    const size_t lds = merge + sizeof(int) * (2 * static_cast<size_t>(sh.S) + 1);
+    const dim3 grid(static_cast<unsigned>(need.teams * need.TS));
+    const dim3 block(64 * kTeamWaves);
+    hipError_t err = sh.D == 128 ? launch(paged_team_kernel<128>, grid, block, lds, stream, a)
+                                 : launch(paged_team_kernel<64>, grid, block, lds, stream, a);
     if (err != hipSuccess) return launched(err, who);
-    PStreamReduceArgs r{};
+    TeamReduceArgs r{};
     r.out = a.out;
-    r.ws_max = a.ws_max;
-    r.ws_sum = a.ws_sum;
-    r.ws_out = a.ws_out;
     r.frag = a.frag;
     r.meta = a.meta;
     r.H = a.H;
     r.G = a.G;
     r.nhc = a.nhc;
-    r.MP = a.MP;
-    r.part_blocks = a.part_blocks;
+    r.TS = need.TS;
     r.gstride = std::min(16, a.G);
-    r.TS = a.Hkv * a.nhc;
-    // Partition slots and boundary slots: at most MP + (MP - 1) fragments
-    // per head when every partition holds a boundary.
-    const dim3 rgrid((a.H + 3) / 4, sh.S);
-    if (2 * a.MP - 1 <= kReduceSmall) {
-        err = sh.D == 128 ? launch(paged_reduce_pstream_wave_kernel<128, kReduceSmall>, rgrid, dim3(256), 0, stream, r)
-                          : launch(paged_reduce_pstream_wave_kernel<64, kReduceSmall>, rgrid, dim3(256), 0, stream, r);
-    } else {
-        const dim3 sgrid(a.H, sh.S);
-        err = sh.D == 128 ? launch(paged_reduce_pstream_split_kernel<128>, sgrid, dim3(256), 0, stream, r)
-                          : launch(paged_reduce_pstream_split_kernel<64>, sgrid, dim3(256), 0, stream, r);
-    }
+    const dim3 rgrid(a.H, sh.S);
+    err = sh.D == 128 ? launch(paged_team_reduce_kernel<128>, rgrid, dim3(256), 0, stream, r)
+                      : launch(paged_team_reduce_kernel<64>, rgrid, dim3(256), 0, stream, r);
     return launched(err, who);
 }
 
@@ -1774,7 +1599,19 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
         }
         if ((rc = require_device()) != SWIFTLLM_OK) return rc;
         if (sh.S == 0) return ok();
-        return decode_balanced(out, ws, ws_bytes, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
+        const StreamNeed need = stream_need(sh, device_cus());
+        if (ws_bytes < need.total) {
+            return fail(SWIFTLLM_ERR_INVALID_PARAMETER, "%s: workspace of %zu bytes, %zu needed", who,
+                        ws_bytes, need.total);
+        }
+        if (single_pass(sh, device_cus())) {
+            return decode_v1(out, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
+        }
+        const TeamNeed team = team_need(sh, device_cus());
+        if (team.teams > 0 && team.total <= need.total) {
+            return decode_team(out, ws, q, kc, vc, bt, ctx, scale, sh, num_blocks, team, stream, who);
+        }
+        return decode_balanced(out, ws, need, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
     }
     const V2Need need = v2_need(sh, partition_size, device_cus());
     if (sh.S > 0) {
@@ -1788,6 +1625,13 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
     }
     if ((rc = require_device()) != SWIFTLLM_OK) return rc;
     if (sh.S == 0) return ok();
+    if (single_pass(sh, device_cus())) {
+        return decode_v1(out, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
+    }
+    const TeamNeed team = team_need(sh, device_cus());
+    if (team.teams > 0 && team.total <= need.total) {
+        return decode_team(out, ws, q, kc, vc, bt, ctx, scale, sh, num_blocks, team, stream, who);
+    }
     DecodeArgs a = make_args(out, q, kc, vc, bt, ctx, scale, sh, num_blocks);
     char* base = static_cast<char*>(ws);
     a.ws_max = reinterpret_cast<float*>(base);
@@ -1795,7 +1639,7 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
     a.ws_out = reinterpret_cast<float*>(base + 2 * need.stat);
     a.part_blocks = partition_size / kBlockTokens;
     a.MP = need.MP;
-    if (need.pstream) return decode_pstream(a, base, need, sh, stream, who);
+    a.share = item_share(a);
     bool too_large = false;
     hipError_t err = launch_partition<kWavesV2>(a, sh.D, stream, &too_large);
     if (too_large) {
@@ -1809,10 +1653,12 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
     r.ws_max = a.ws_max;
     r.ws_sum = a.ws_sum;
     r.ws_out = a.ws_out;
+    r.S = a.S;
     r.H = a.H;
     r.MB = a.MB;
     r.part_blocks = a.part_blocks;
     r.MP = a.MP;
+    r.share = a.share;
     err = sh.D == 128 ? launch_reduce_t<128>(r, sh.S, stream)
                       : launch_reduce_t<64>(r, sh.S, stream);
     return launched(err, who);

@@ -477,3 +477,74 @@ def test_partition_stream_reduce_fragment_counts(dev, D):
     live = lens > 0
     assert np.all(out[~live] == 0), "empty sequences must be zero"
     assert_attention_close(out[live], _ref(w)[live], f"reduce fragment counts D{D}")
+
+
+def _padded(w, mb):
+    """The same batch with block tables mb wide (the width is what the
+    launcher sees of the lengths)."""
+    bt = np.zeros((w.block_tables.shape[0], mb), np.int32)
+    bt[:, :w.block_tables.shape[1]] = w.block_tables
+    return workloads.DecodeWorkload("padded", w.q, w.key_cache, w.value_cache, bt, w.context_lens,
+                                    w.scale)
+
+
+@pytest.mark.parametrize("H,Hkv,D,S", [
+    (32, 8, 128, 1), (32, 8, 128, 7), (64, 8, 128, 40), (8, 8, 64, 128),  # teams: up to 2 sequences each
+    (8, 8, 64, 129),                       # one more: items
+    (48, 2, 128, 5), (16, 1, 64, 300),     # two head chunks, the second 8 wide; one-member teams
+    (128, 128, 64, 8), (256, 256, 64, 3),  # 4 teams; too few: items / streams
+])
+def test_split_routes_agree_with_single_pass(dev, H, Hkv, D, S):
+    """Tables padded past every single-pass limit send split-K calls to the
+    teams (few sequences) or the item list (many), narrow ones to the single
+    pass; all against the oracle, with empty, one-token and block-edge
+    contexts, NaN in unused slots and an out-of-pool block."""
+    rng = np.random.default_rng(H + 7 * Hkv + D + S)
+    lens = np.clip(np.rint(np.exp(rng.normal(np.log(120.0), 1.2, size=S))), 0, 900).astype(np.int64)
+    edge = np.array([0, 1, 15, 16, 17, 900])[:max(S - 1, 0)]
+    lens[:len(edge)] = edge
+    if S == 1:
+        lens[:] = 777
+    w = _random_batch(rng, lens, H, Hkv, D)
+    for s in range(S):
+        if lens[s] % 16:
+            b = w.block_tables[s, lens[s] // 16]
+            w.key_cache[b, :, :, lens[s] % 16:] = np.nan
+            w.value_cache[b, :, :, lens[s] % 16:] = np.nan
+    ref = _ref(w)
+    live = lens > 0
+    for mb in (w.block_tables.shape[1], 3000):
+        dw = DeviceWorkload(_padded(w, mb))
+        for variant, ps in (("v1", None), ("v2", 16), ("v2", 512), ("v2", 0)):
+            out = dw.run(variant, partition_size=ps)
+            assert np.all(out[~live] == 0), f"MB={mb} {variant} {ps}: empty sequences must be zero"
+            assert_attention_close(out[live], ref[live], f"H{H}/{Hkv} D{D} S{S} MB={mb} {variant} ps={ps}")
+
+
+@pytest.mark.parametrize("ps", [16, 64, 512])
+def test_items_of_several_partitions(dev, ps):
+    """More sequences than teams, long tables: an item takes several
+    partitions of the batch, and the reduce has to cut the sequences the same
+    way; up to 188 partitions per sequence (the four-wave reduce) and 6 (one
+    wave)."""
+    rng = np.random.default_rng(19 + ps)
+    S = 140
+    lens = np.clip(np.rint(np.exp(rng.normal(np.log(500.0), 1.2, size=S))), 1, 3000).astype(np.int64)
+    lens[:4] = [0, 1, 3000, 2999]
+    w = _random_batch(rng, lens, H=32, Hkv=8, D=64)
+    out = DeviceWorkload(w).run("v2", partition_size=ps)
+    live = lens > 0
+    assert np.all(out[~live] == 0)
+    assert_attention_close(out[live], _ref(w)[live], f"items ps={ps}")
+
+
+@pytest.mark.parametrize("counts", [(1, 2, 63, 64), (16, 17, 4, 129)])
+def test_team_fragment_counts(dev, counts):
+    """Sequences whose blocks span 1 to all 64 teams of an 8-kv-head batch
+    (ranges that end on, before and after a sequence's end)."""
+    rng = np.random.default_rng(sum(counts))
+    lens = np.array([16 * c - (i % 3) * 5 for i, c in enumerate(counts)])
+    w = _padded(_random_batch(rng, lens, H=64, Hkv=8, D=128), 3000)
+    dw = DeviceWorkload(w)
+    for ps in (512, 0):
+        assert_attention_close(dw.run("v2", partition_size=ps), _ref(w), f"teams {counts} ps={ps}")
