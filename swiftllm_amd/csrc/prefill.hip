@@ -33,7 +33,12 @@
 // unit's workgroups latest tokens first (the longest walks start first), so
 // the workgroups resident on an XCD share one unit's K/V in its L2. K/V tiles are loaded
 // with ordinary (cached) loads: every query group of a sequence re-reads them.
+//
+// That kernel serves negative and zero scales, caches that are not 16-byte
+// aligned and batches of more than 1024 prompts; the usual call takes
+// paged_prefill_shared_kernel (below), whose waves share their stages.
 
+#include <algorithm>
 #include <type_traits>
 #include "attention_core.hpp"
 
@@ -62,6 +67,8 @@ struct PrefillArgs {
     int groups;          // workgroups per (sequence, kv head chunk) in the grid
     long long units;     // (sequence, kv head chunk) pairs: S * Hkv * nhc
     int num_blocks;      // bound on block ids; <= 0: unbounded
+    bool q16, out16;     // shared stages: q and out are 16-byte aligned
+    int xcds;            // shared stages: XCDs the kv heads are dealt over, 8 or 1
 };
 
 // FOLD: scale_log2 > 0 (the usual 1/sqrt(D)), whose scale then goes into the
@@ -491,6 +498,498 @@ void paged_prefill_kernel(const PrefillArgs a) {
     store(sb, ok_b, qrow_b);
 }
 
+// ---------------------------------------------------------------------------
+// Shared stages: the prefill kernel for positive scales and 16-byte aligned
+// caches, up to kSharedMaxSeqs sequences.
+//
+// A workgroup's four waves take consecutive tokens of one kv head, so they
+// walk the same keys: each stage of 64 keys (four blocks) goes into LDS once
+// for all of them, one block per wave by direct buffer loads, two stages
+// deep, one barrier a stage. A wave owns 32 query rows (32 / gw tokens x gw =
+// min(G, 32) heads) on v_mfma_f32_32x32x16_f16: S^T = K Q^T leaves a lane 32
+// scores of one query row, so a row's maximum and sum are in-lane up to one
+// lane swap, and P goes into PV straight from those registers. V lies in the
+// cache as that product's row operand already; K comes back transposed by
+// ds_read_b64_tr_b16, with its rows permuted so that both operands of PV are
+// contiguous. The next stage's scores are made among this stage's weights.
+//
+// Work list. Every workgroup of a resident grid walks a list of query tiles,
+// longest walk first over all sequences, each XCD its own kv heads, so no
+// slot is left with a long tile at the end and no empty workgroup is launched
+// for short prompts. Outputs go through LDS as whole rows, nontemporally.
+//
+// Bound: MFMA, at the clock the power limit leaves. On 8 x 2048 tokens the
+// matrix pipes are busy 51% of the cycles at 1.75 GHz, on 1 x 8192 58% at
+// 1.65 GHz (32/8 heads x 128): 1.12 PFLOP/s with the lo half of P, where
+// operands in registers alone reach 1.6. Fewer VALU instructions (the lo half
+// by mixed-precision multiply-adds), other interleavings of MFMA and VALU and
+// wave priorities moved it by under 3% either way. Measured on one box
+// (us per call, per-wave tiles -> this kernel): 8 x 2048 545 -> 443, 1 x 8192
+// 887 -> 734, 1 x 2048 82 -> 66, 24 prompts of 1-2457 tokens 241 -> 190, 64
+// of 16-200 60.8 -> 41.2, 4 x 1000-3000 of 16/16 heads 217 -> 157, 8 x 2048
+// of 8/8 heads x 64 101 -> 66, 1 x 17 7.0 -> 7.1. Of that, tiles longest first
+// against sequence by sequence: 208 -> 196 (24 prompts), 190 -> 165 (16/16
+// heads), 88 -> 70 (x 64); whole-row outputs 54 -> 43 (64 short prompts).
+// Loading the next tile's first stages and Q during a tile's last stage
+// changed nothing (459 -> 470, 55 -> 55) and is not done.
+// ---------------------------------------------------------------------------
+constexpr int kSharedMaxSeqs = 1024;  // sequences in the LDS tile table
+constexpr long long kSharedCUs = 256;  // MI355X; any grid is correct, this one is resident at once
+template <int D>
+constexpr int kSharedPerCU = D == 128 ? 2 : 3;  // workgroups per CU, waves per SIMD
+
+typedef float f16x __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f16x mfma32(h8 a, h8 b, f16x c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// LDS of one stage (64 keys), in halves: four K tiles [d][16], then four V
+// tiles in operand order. The second K tile of a pair sits 128 bytes off, so
+// that the two tiles' rows an operand read takes together fall in different
+// banks.
+template <int D>
+struct Stage {
+    static constexpr int kTile = D * kBlockTokens;
+    static constexpr int kOdd = kTile + 64;
+    static constexpr int kPair = 2 * kTile + 128;
+    static constexpr int kK = 2 * kPair;
+    static constexpr int kV = 4 * kTile;
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const f16* cache, int b, int kvh, int Hkv, int D) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<f16*>(cache + kv_tile_offset(b, kvh, Hkv, D)), 0,
+                                             D * kBlockTokens * 2, kRsrcWord3);
+}
+
+// Block b's K tile into its place of a K stage, copied as it is.
+template <int D>
+__device__ __forceinline__ void stage_k(const PrefillArgs& a, f16* ks, int w, int b, int kvh, int lane) {
+    const __amdgpu_buffer_rsrc_t rk = tile_rsrc(a.kc, b, kvh, a.Hkv, D);
+    f16* const k = ks + (w >> 1) * Stage<D>::kPair + (w & 1) * Stage<D>::kOdd;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to_lds(k + 512 * i), 16, 16u * lane, 1024u * i, 0, 0);
+    }
+}
+
+// Block b's V tile into its place of a V stage, each 32-row piece's 16-byte
+// chunks in operand order: the rows' first 8 tokens, then their last 8.
+template <int D>
+__device__ __forceinline__ void stage_v(const PrefillArgs& a, f16* vs, int w, int b, int kvh, int lane) {
+    const __amdgpu_buffer_rsrc_t rv = tile_rsrc(a.vc, b, kvh, a.Hkv, D);
+    f16* const v = vs + w * Stage<D>::kTile;
+    const unsigned vo = 32u * (lane & 31) + 16u * (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to_lds(v + 512 * i), 16, vo, 1024u * i, 0, 0);
+    }
+}
+
+// Zeroes tokens nv .. 15 of the wave's V tile in LDS, once its loads have
+// landed: stale values there (perhaps NaN) have weight 0.
+template <int D>
+__device__ __forceinline__ void clean_v(f16* vs, int w, int nv, int lane) {
+    const int n = min(max(nv - 8 * (lane >> 5), 0), 8);
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+        h8* const p = reinterpret_cast<h8*>(vs + w * Stage<D>::kTile + 512 * i + 8 * lane);
+        h8 v = *p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = e < n ? v[e] : static_cast<f16>(0.0f);
+        *p = v;
+    }
+}
+
+// S^T of a 64-key stage: sc[T] the 32 keys of pair T.
+template <int D>
+__device__ __forceinline__ void qk_stage(f16x (&sc)[2], const f16* kl, const h8 (&q)[D / 16]) {
+    sc[0] = f16x{};
+    sc[1] = f16x{};
+#pragma unroll
+    for (int J = 0; J < D / 16; ++J) {
+#pragma unroll
+        for (int T = 0; T < 2; ++T) {
+            const f16* p = kl + T * Stage<D>::kPair + 256 * J;
+            const s4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(const_cast<f16*>(p)));
+            const s4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(const_cast<f16*>(p + 64)));
+            sc[T] = mfma32(cat8(__builtin_bit_cast(h4, x), __builtin_bit_cast(h4, y)), q[J], sc[T]);
+        }
+    }
+}
+
+// Query tiles (per_wg tokens) and token prefix of every sequence: of up to 64
+// sequences in registers, one per lane (no barrier before the first tile), of
+// more in LDS.
+struct TileLds {
+    int tiles[kSharedMaxSeqs];
+    int start[kSharedMaxSeqs];  // tokens before the sequence
+};
+
+struct TileTable {
+    TileLds* lds;  // S > 64
+    int S;
+    int tiles;     // S <= 64: of sequence `lane`
+    int start;
+    __device__ __forceinline__ int tiles_of(int s0, int lane) const {
+        if (S <= 64) return tiles;
+        return s0 + lane < S ? lds->tiles[s0 + lane] : 0;
+    }
+    __device__ __forceinline__ int start_of(int s) const {
+        return __builtin_amdgcn_readfirstlane(S <= 64 ? __builtin_amdgcn_readlane(start, s) : lds->start[s]);
+    }
+    // (tile, sequence) pairs with a tile index >= i.
+    __device__ __forceinline__ int count(int i, int lane) const {
+        int n = 0;
+        for (int s0 = 0; s0 < S; s0 += 64) n += max(tiles_of(s0, lane) - i, 0);
+        return wave_total(n);
+    }
+};
+
+__device__ __forceinline__ TileTable make_tiles(const int* ctx, int S, int per_wg, int max_tiles, TileLds* lds,
+                                                int* s_part) {
+    TileTable t{lds, S, 0, 0};
+    const int lane = threadIdx.x & 63;
+    if (S <= 64) {
+        const int len = lane < S ? max(ctx[lane], 0) : 0;
+        t.tiles = min((len + per_wg - 1) / per_wg, max_tiles);
+        t.start = wave_inclusive_scan(len) - len;
+        return t;
+    }
+    constexpr int kEach = kSharedMaxSeqs / (64 * kPrefillWaves);
+    const int c0 = threadIdx.x * kEach;
+    int len[kEach];
+    int sum = 0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        len[i] = c0 + i < S ? max(ctx[c0 + i], 0) : 0;
+        sum += len[i];
+    }
+    const int incl = wave_inclusive_scan(sum);
+    const int w = threadIdx.x >> 6;
+    if (lane == 63) s_part[w] = incl;
+    __syncthreads();
+    int at = incl - sum;
+    for (int i = 0; i < w; ++i) at += s_part[i];
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        if (c0 + i < S) {
+            lds->tiles[c0 + i] = min((len[i] + per_wg - 1) / per_wg, max_tiles);
+            lds->start[c0 + i] = at;
+            at += len[i];
+        }
+    }
+    __syncthreads();
+    return t;
+}
+
+// Entry e (below count(0)) of the list of (tile, sequence) pairs, highest tile
+// index (longest walk) first, sequences in order within one index. Every wave
+// works it out for itself.
+__device__ __forceinline__ void nth_tile(const TileTable& tt, int max_tiles, int e, int lane, int& tile, int& seq) {
+    int lo = 0, hi = max_tiles, below = 0;  // count(lo) > e >= count(hi) = below
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        const int n = tt.count(mid, lane);
+        if (n > e) {
+            lo = mid;
+        } else {
+            hi = mid;
+            below = n;
+        }
+    }
+    tile = lo;
+    int k = e - below;  // the k-th sequence with more than `lo` tiles
+    for (int s0 = 0;; s0 += 64) {
+        const bool has = tt.tiles_of(s0, lane) > lo;
+        const unsigned long long mask = __ballot(has);
+        const int n = __popcll(mask);
+        if (k < n || s0 + 64 >= tt.S) {
+            const int rank = __popcll(mask & ((1ull << lane) - 1ull));
+            seq = s0 + __ffsll(static_cast<long long>(__ballot(has && rank == k))) - 1;
+            return;
+        }
+        k -= n;
+    }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kPrefillWaves) __attribute__((amdgpu_waves_per_eu(kSharedPerCU<D>)))
+void paged_prefill_shared_kernel(const PrefillArgs a) {
+    constexpr int NJ = D / 16;   // 16-wide k steps of QK^T
+    constexpr int ND = D / 32;   // 32-row pieces of the output
+    using St = Stage<D>;
+    __shared__ int s_part[kPrefillWaves];
+    __shared__ TileLds s_tiles;
+    __shared__ __align__(16) f16 s_k[2][St::kK];
+    __shared__ __align__(16) f16 s_v[2][St::kV];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int per_wg = kPrefillWaves * a.tpw;
+    const TileTable tt = make_tiles(a.ctx, a.S, per_wg, a.groups, &s_tiles, s_part);
+
+    // Query row r of the wave in a tile: token tq0 + r / gw, head r % gw.
+    const int r = lane & 31;
+    const int h = lane >> 5;
+    // K operand: lane (16-lane group g4, j) reads 4 tokens of row j / 4 of
+    // its 4-row piece; ds_read_b64_tr_b16 hands lane j the piece's 4 rows of
+    // one token. Groups 0 and 2 take the pair's first block, 1 and 3 its
+    // second, groups 2 and 3 the upper 8 of the 16 rows. The tokens of j / 4
+    // = 1 and 2 are exchanged, so the products' rows 8 a + 4 h + c hold the
+    // block's tokens 8 h + 4 a + c: a lane's eight scores of a block are then
+    // eight consecutive tokens, and its V operand 16 contiguous bytes.
+    const int g4 = lane >> 4;
+    const int j = lane & 15;
+    const int swapped = ((j & 1) << 1) | ((j >> 1) & 1);
+    const int koff = (g4 & 1) * St::kOdd + (8 * (g4 >> 1) + (j >> 2)) * kBlockTokens + 4 * swapped;
+
+    // Workgroups go to the 8 XCDs round-robin, so blockIdx.x % xcds names the
+    // XCD (xcds is 1 when the kv heads do not divide over them). Each XCD runs
+    // every sequence's tiles of its own kv heads, so a unit's K/V is read
+    // through one L2. Its workgroups take the list in rounds, every other one
+    // backwards.
+    const unsigned x = blockIdx.x % a.xcds;
+    const unsigned l0 = blockIdx.x / a.xcds;
+    const unsigned wgs = gridDim.x / a.xcds;
+    const unsigned heads = a.Hkv * a.nhc / a.xcds;
+    const unsigned total = static_cast<unsigned>(tt.count(0, lane)) * heads;  // below 2^31 (host)
+    auto item_of = [&](unsigned round) { return round * wgs + ((round & 1) ? wgs - 1 - l0 : l0); };
+    for (unsigned round = 0; item_of(round) < total; ++round) {
+    if (round > 0) __syncthreads();  // the stages are free for the next tile
+    const unsigned item = item_of(round);
+    const unsigned e = item / heads;
+    int tile, s;
+    nth_tile(tt, a.groups, static_cast<int>(e), lane, tile, s);
+    s = __builtin_amdgcn_readfirstlane(s);
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    const int yy = static_cast<int>(x + a.xcds * (item - e * heads));
+    const int kvh = yy / a.nhc;
+    const int hc = yy - kvh * a.nhc;
+    const int start = tt.start_of(s);
+    const int L = max(as_const(a.ctx)[s], 0);
+    const int wg_last = min((tile + 1) * per_wg, L) - 1;
+    const int nkb = wg_last / kBlockTokens + 1;
+    const int nsteps = wg_last / 64 + 1;
+    // (worked out per tile behind an empty asm, so that neither stays in a
+    // register through the walk)
+    int rr = r;
+    asm volatile("" : "+v"(rr));
+    const int rt = rr / a.gw;
+    const int rh = rr - rt * a.gw;
+    const int g = hc * 32 + rh;
+    const int head = kvh * a.G + min(g, a.G - 1);
+    const int tq0 = tile * per_wg + w * a.tpw;
+    const int tq = tq0 + rt;
+    const bool ok = (rt < a.tpw) && (g < a.G) && tq < L;
+    const size_t qrow = (static_cast<size_t>(start) + min(tq, L - 1)) * a.H + head;
+    const int lim = ok ? tq + 1 : 0;                  // keys this row sees
+    const int rel = ok ? rt * a.H + head : -1;        // row among the wave's tokens
+
+    const const_int* srow = as_const(a.slots) + start;
+    auto chunk_ids = [&](int c) {
+        return srow[static_cast<size_t>(min(64 * c + lane, nkb - 1)) * kBlockTokens] >> kBlockShift;
+    };
+    int ids = chunk_ids(0);
+    int ids_next = chunk_ids(1);
+    // Q^T operand: lane (r, h) holds q[r][16 J + 8 h .. + 7].
+    h8 q[NJ];
+    {
+        const f16* p = a.q + qrow * D + 8 * h;
+        if (a.q16) {
+#pragma unroll
+            for (int J = 0; J < NJ; ++J) q[J] = *reinterpret_cast<const h8*>(p + 16 * J);
+        } else {
+#pragma unroll
+            for (int J = 0; J < NJ; ++J) {
+                q[J] = cat8(*reinterpret_cast<const h4*>(p + 16 * J), *reinterpret_cast<const h4*>(p + 16 * J + 4));
+            }
+        }
+#pragma unroll
+        for (int J = 0; J < NJ; ++J) q[J] = ok ? q[J] : h8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    // Block of this wave in stage u (stages asked for in order) and, in ok4,
+    // which of the stage's four blocks are in the pool.
+    auto block_of = [&](int u, int& ok4) {
+        if (u > 0 && (u & 15) == 0) {
+            ids = ids_next;
+            ids_next = chunk_ids((u >> 4) + 1);
+        }
+        const unsigned long long okm = __ballot(block_ok(ids, a.num_blocks));
+        const int at = 4 * (u & 15);
+        ok4 = static_cast<int>((okm >> at) & 15ull);
+        const int b = __builtin_amdgcn_readlane(ids, at + w);
+        return block_ok(b, a.num_blocks) ? b : 0;
+    };
+
+    f16x acc[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) acc[i] = f16x{};
+    float m = -INFINITY, l = 0.0f;
+
+    // Tokens of this wave's block of stage u that exist.
+    auto tokens_of = [&](int u, int ok4) {
+        return ((ok4 >> w) & 1) ? min(max(L - (64 * u + 16 * w), 0), kBlockTokens) : 0;
+    };
+    int ok_t, ok_1, ok_2 = 15;  // of stages t, t + 1 and t + 2
+    int b_1 = 0, b_2 = 0;
+    {
+        const int b = block_of(0, ok_t);
+        stage_k<D>(a, s_k[0], w, b, kvh, lane);
+        stage_v<D>(a, s_v[0], w, b, kvh, lane);
+        ok_1 = 15;
+        if (nsteps > 1) {
+            b_1 = block_of(1, ok_1);
+            stage_k<D>(a, s_k[1], w, b_1, kvh, lane);
+        }
+        wait_vm<0>();
+        const int nv = tokens_of(0, ok_t);
+        if (nv < kBlockTokens) clean_v<D>(s_v[0], w, nv, lane);
+    }
+    __syncthreads();
+    f16x sc[2];
+    qk_stage<D>(sc, s_k[0] + koff, q);
+    __syncthreads();
+    // Stage t; kMore: another follows, and its scores are made among this one's
+    // weights.
+    auto step = [&](auto more, int t) {
+        constexpr bool kMore = decltype(more)::value;
+        if constexpr (kMore) {
+            stage_v<D>(a, s_v[(t + 1) & 1], w, b_1, kvh, lane);
+            if (t + 2 < nsteps) {
+                b_2 = block_of(t + 2, ok_2);
+                stage_k<D>(a, s_k[t & 1], w, b_2, kvh, lane);
+            }
+        }
+        const int base = 64 * t;
+        {
+            // Score i of tile T: key base + 32 T + 16 (i / 8) + 8 h + i % 8.
+            if (base + 63 > tq0 || ok_t != 15) [[unlikely]] {
+#pragma unroll
+                for (int T = 0; T < 2; ++T) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int key = base + 32 * T + 16 * (i >> 3) + 8 * h + (i & 7);
+                        if (key >= lim || !((ok_t >> (2 * T + (i >> 3))) & 1)) sc[T][i] = -INFINITY;
+                    }
+                }
+            }
+            float bm = max3(max3(sc[0][0], sc[0][1], sc[0][2]), max3(sc[0][3], sc[0][4], sc[0][5]), sc[0][6]);
+#pragma unroll
+            for (int i = 7; i < 31; i += 2) bm = max3(bm, sc[i >> 4][i & 15], sc[(i + 1) >> 4][(i + 1) & 15]);
+            bm = max2(bm, sc[1][15]);
+            {
+                float x, y;
+                swap32(bm, x, y);
+                bm = max2(x, y) * a.scale_log2;
+            }
+            if (__any(bm > m + kLazyMargin)) {
+                const float m_new = fmaxf(m, bm);
+                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+#pragma unroll
+                for (int i = 0; i < ND; ++i) acc[i] *= alpha;
+                l *= alpha;
+                m = m_new;
+            }
+            const float c = ((m == -INFINITY) ? 0.0f : m) - kPExpLazy;
+            f16x sn[2];
+            if constexpr (kMore) qk_stage<D>(sn, s_k[(t + 1) & 1] + koff, q);
+            const f16* const vl = s_v[t & 1] + 8 * lane;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                float p[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b >> 1][8 * (b & 1) + i], a.scale_log2, -c));
+                }
+                l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+                h2 hh[4], ll[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    hh[i] = __builtin_amdgcn_cvt_pkrtz(p[2 * i], p[2 * i + 1]);
+                    ll[i] = __builtin_amdgcn_cvt_pkrtz(sub_h2_lo(p[2 * i], hh[i]), sub_h2_hi(p[2 * i + 1], hh[i]));
+                }
+                const h8 ph = __builtin_bit_cast(h8, __builtin_shufflevector(
+                    __builtin_shufflevector(hh[0], hh[1], 0, 1, 2, 3), __builtin_shufflevector(hh[2], hh[3], 0, 1, 2, 3),
+                    0, 1, 2, 3, 4, 5, 6, 7));
+                const h8 pl = __builtin_bit_cast(h8, __builtin_shufflevector(
+                    __builtin_shufflevector(ll[0], ll[1], 0, 1, 2, 3), __builtin_shufflevector(ll[2], ll[3], 0, 1, 2, 3),
+                    0, 1, 2, 3, 4, 5, 6, 7));
+                h8 v[ND];
+#pragma unroll
+                for (int i = 0; i < ND; ++i) v[i] = *reinterpret_cast<const h8*>(vl + b * St::kTile + 512 * i);
+#pragma unroll
+                for (int i = 0; i < ND; ++i) acc[i] = mfma32(v[i], ph, acc[i]);
+#pragma unroll
+                for (int i = 0; i < ND; ++i) acc[i] = mfma32(v[i], pl, acc[i]);
+            }
+            if constexpr (kMore) {
+                sc[0] = sn[0];
+                sc[1] = sn[1];
+            }
+        }
+        if constexpr (kMore) {
+            wait_vm<0>();
+            const int nv = tokens_of(t + 1, ok_1);
+            if (nv < kBlockTokens) clean_v<D>(s_v[(t + 1) & 1], w, nv, lane);
+            ok_t = ok_1;
+            ok_1 = ok_2;
+            b_1 = b_2;
+            __syncthreads();
+        }
+    };
+    int t = 0;
+    for (; t + 1 < nsteps; ++t) step(std::true_type{}, t);
+    step(std::false_type{}, t);
+
+    // The wave's output rows, through its quarter of the K buffers (every
+    // wave's last scores are made): chunk c (8 values) of row r at chunk
+    // c ^ (r % (D / 8)), so that neither side conflicts, and back as whole rows,
+    // D / 8 lanes each.
+    {
+        float y0, y1;
+        swap32(l, y0, y1);
+        const float sum = y0 + y1;
+        const float inv = (sum > 0.0f) ? 1.0f / sum : 0.0f;
+        constexpr int kChunks = D / 8;
+        f16* const o_lds = &s_k[0][0] + w * 32 * D;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                h4 o;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[c] = static_cast<f16>(acc[i][4 * k + c] * inv);
+                *reinterpret_cast<h4*>(o_lds + r * D + 8 * ((4 * i + k) ^ (r & (kChunks - 1))) + 4 * h) = o;
+            }
+        }
+        f16* const op = a.out + (static_cast<size_t>(start) + tq0) * a.H * D + 8 * (lane & (kChunks - 1));
+        int to[D / 16];
+        h8 v[D / 16];
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) {
+            const int row = (64 / kChunks) * i + lane / kChunks;
+            to[i] = __shfl(rel, row);
+            v[i] = *reinterpret_cast<const h8*>(o_lds + row * D + 8 * ((lane ^ row) & (kChunks - 1)));
+        }
+        if (a.out16) {
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+                if (to[i] >= 0) __builtin_nontemporal_store(v[i], reinterpret_cast<h8*>(op + static_cast<size_t>(to[i]) * D));
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < D / 16; ++i) {
+                h4* const o = reinterpret_cast<h4*>(op + static_cast<size_t>(to[i]) * D);
+                if (to[i] >= 0) {
+                    o[0] = __builtin_shufflevector(v[i], v[i], 0, 1, 2, 3);
+                    o[1] = __builtin_shufflevector(v[i], v[i], 4, 5, 6, 7);
+                }
+            }
+        }
+    }
+    }
+}
+
 int prefill(const char* who, void* out, const void* q, const void* kc, const void* vc,
             const int* slots, const int* ctx, float scale, long long S, long long H, long long Hkv,
             long long D, long long BS, long long max_len, int num_blocks, hipStream_t stream) {
@@ -556,6 +1055,24 @@ int prefill(const char* who, void* out, const void* q, const void* kc, const voi
                     static_cast<unsigned>((rounds + gy - 1) / gy));
     const dim3 block(64 * kPrefillWaves);
     const bool fold = a.scale_log2 > 0.0f;
+    const int wide_gw = a.G < 32 ? a.G : 32;
+    const int wide_heads = a.Hkv * ((a.G + 31) / 32);
+    const long long wide_per = static_cast<long long>(kPrefillWaves) * (32 / wide_gw);
+    const long long items = S * wide_heads * ((max_len + wide_per - 1) / wide_per);
+    if (fold && S <= kSharedMaxSeqs && items < (1LL << 30) && aligned(kc, 16) && aligned(vc, 16)) {
+        a.nhc = (a.G + 31) / 32;
+        a.gw = wide_gw;
+        a.tpw = 32 / wide_gw;
+        a.groups = static_cast<int>((max_len + wide_per - 1) / wide_per);
+        const int heads = wide_heads;
+        a.xcds = heads % 8 == 0 ? 8 : 1;
+        a.q16 = aligned(q, 16);
+        a.out16 = aligned(out, 16);
+        const long long wgs = std::min<long long>((items + 7) / 8 * 8, kSharedCUs * (D == 128 ? kSharedPerCU<128> : kSharedPerCU<64>));
+        return launched(launch(D == 128 ? paged_prefill_shared_kernel<128> : paged_prefill_shared_kernel<64>,
+                               dim3(static_cast<unsigned>(wgs)), block, 0, stream, a),
+                        who);
+    }
     const bool ldsk = aligned(kc, 16);
     using K = void (*)(PrefillArgs);
     static const K kernels[2][2][2] = {

@@ -203,3 +203,50 @@ def test_paged_attention_prefill_op(dev):
     assert_attention_close(out.numpy().reshape(B * S, H, D), _ref(w), "PagedAttention.prefill")
     b, o = w.slot_mapping // 16, w.slot_mapping % 16
     assert np.array_equal(kc.numpy()[b, :, :, o].view(np.uint16), w.key.view(np.uint16))
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(8, 8, 128), (6, 2, 64), (10, 2, 128), (24, 1, 128), (40, 1, 64),
+                                     (66, 2, 128), (32, 16, 64)])
+def test_prefill_tiles_around_stage_ends(dev, H, Hkv, D):
+    """Rows per wave of 32 tokens x 1 head to 1 token x 32 heads (and chunks of
+    32 heads whose second is 8 or 1 wide), kv heads that do and do not divide
+    over the 8 XCDs, prompts that end on, before and after a 64-key stage, and
+    walks past one and two chunks of 64 block ids."""
+    lens = (63, 64, 65, 0, 127, 128, 129, 1023, 1024, 1041, 1, 2100)
+    if H * D > 4096:
+        lens = (63, 64, 65, 0, 129, 1, 1041)
+    w = workloads.prefill_config(lens, H, Hkv, D, seed=H + Hkv + D)
+    assert_attention_close(_run(w, max_len=5000), _ref(w), f"prefill tiles H{H} Hkv{Hkv} D{D}")
+
+
+@pytest.mark.parametrize("S,top", [(64, 300), (65, 300), (1024, 40), (1025, 40)])
+def test_prefill_tile_list(dev, S, top):
+    """Sequence counts around the register and LDS tables of the work list and
+    its limit, with more tiles than the grid holds workgroups and many prompts
+    of equal length."""
+    rng = np.random.default_rng(S)
+    lens = rng.integers(0, top, size=S)
+    lens[rng.choice(S, size=S // 4, replace=False)] = top
+    w = workloads.prefill_config(lens, 8, 8, 64, seed=S)
+    assert_attention_close(_run(w), _ref(w), f"prefill S={S}")
+
+
+@pytest.mark.parametrize("shift", ["q", "out", "value_cache"])
+def test_prefill_8_byte_aligned_arrays(dev, shift):
+    """q, out or the value cache 8 bytes past a 16-byte boundary."""
+    w = workloads.prefill_config((1, 17, 70, 129), 32, 8, 128, seed=17)
+    T, H, D = w.q.shape
+    arrays = {"q": w.q, "out": np.full_like(w.q, np.nan), "key_cache": w.key_cache,
+              "value_cache": w.value_cache}
+    bufs = {k: DeviceArray((a.size + 8,), np.float16) for k, a in arrays.items()}
+    at = {k: 8 if k == shift else 0 for k in arrays}
+    for k, a in arrays.items():
+        bufs[k].upload_at(at[k], a)
+    p = {k: bufs[k].ptr + at[k] for k in arrays}
+    sm, ctx = DeviceArray.from_numpy(w.slot_mapping), DeviceArray.from_numpy(w.context_lens)
+    pa.launch_paged_prefill(p["out"], p["q"], p["key_cache"], p["value_cache"], sm, ctx, w.scale,
+                            len(w.context_lens), H, 8, D, 16, int(w.context_lens.max()),
+                            num_blocks=w.key_cache.shape[0])
+    synchronize()
+    out = bufs["out"].download_at(at["out"], w.q.shape, np.float16)
+    assert_attention_close(out, _ref(w), f"prefill, {shift} at +8 bytes")
