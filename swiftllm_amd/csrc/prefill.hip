@@ -884,7 +884,9 @@ void paged_prefill_shared_kernel(const PrefillArgs a) {
             }
             if (__any(bm > m + kLazyMargin)) {
                 const float m_new = fmaxf(m, bm);
-                const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+                // A row that has seen no key yet (its blocks are outside the
+                // pool) keeps its zeros: -inf - -inf would make them NaN.
+                const float alpha = (m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
 #pragma unroll
                 for (int i = 0; i < ND; ++i) acc[i] *= alpha;
                 l *= alpha;

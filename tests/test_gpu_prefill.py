@@ -250,3 +250,19 @@ def test_prefill_8_byte_aligned_arrays(dev, shift):
     synchronize()
     out = bufs["out"].download_at(at["out"], w.q.shape, np.float16)
     assert_attention_close(out, _ref(w), f"prefill, {shift} at +8 bytes")
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(8, 8, 64), (8, 8, 128), (8, 4, 128)])
+def test_prefill_first_block_out_of_pool(dev, H, Hkv, D):
+    """The first block of a prompt outside the pool: the rows of a wave's 32
+    that see only that block attend to no key and come out as zeros, beside
+    rows of the same wave that see the next block. The others attend to the
+    keys from position 16 on, as a prompt that starts there would."""
+    L = 90
+    w = workloads.prefill_config((L, 33), H, Hkv, D, seed=31 + D)
+    w.slot_mapping[:16] = -1
+    out = _run(w)
+    assert np.array_equal(out[:16].view(np.uint16), np.zeros((16, H, D), np.uint16))
+    ref = oracle.prefill_numpy(w.q[16:], w.key_cache, w.value_cache, w.slot_mapping[16:],
+                               np.array([L - 16, 33]), w.scale)
+    assert_attention_close(out[16:], ref, f"prefill first block out H{H} Hkv{Hkv} D{D}")
