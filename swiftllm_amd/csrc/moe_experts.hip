@@ -392,7 +392,8 @@ __global__ __launch_bounds__(kThreads) void moe_expert_gemm_kernel(const GemmArg
 constexpr int kThinThreads = 256;   // 4 waves
 constexpr int kThinLds = 160 * 1024;
 
-// Output columns per workgroup: 128 plain (4 waves of 32 columns), 64 gated
+// Output columns per workgroup: 128 plain (4 waves of 32 columns; fewer where
+// that leaves CUs idle, thin_columns below), 64 gated
 // (2 column tiles of 32, each for two waves that share its tail tiles), so
 // that the gated GEMM's n / 64 x E workgroups of a decode batch (1792 for
 // Mixtral's 14336 x 8) fill whole rounds on 256 CUs.
@@ -402,11 +403,11 @@ constexpr int thin_out() { return GATED ? 64 : 128; }
 // A thin tile's shape for a tail of at most 32 NTT rows (NTT = 1, 2 or 4
 // tiles of 32): a stage holds the tile's TW weight rows and 32 NTT tail rows
 // (the last one repeated), and as many stages as fit in the LDS make the
-// ring (8 for NTT = 1, 6 for 2, 5 for 4), so short tails, which load fewer
+// ring (8 for NTT = 1, 6 for 2, 5 for 4 at 128 weight rows), so short tails, which load fewer
 // rows per stage, keep more stages in flight.
-template <bool GATED, int NTT>
+template <bool GATED, int OUT_COLS, int NTT>
 struct Thin {
-    static constexpr int OUT = thin_out<GATED>();
+    static constexpr int OUT = OUT_COLS;
     static constexpr int TW = GATED ? 2 * OUT : OUT;              // weight rows per stage
     static constexpr int ROWS = TW + 32 * NTT;                     // stage rows
     static constexpr int L = ROWS * kRowChunks / kThinThreads;    // loads per thread per stage
@@ -424,11 +425,11 @@ struct Thin {
 // slots j * 256 + wv * 64 + lane (8 rows: tile weight rows, then tail rows).
 // A __device__ function rather than a lambda: a lambda issuing these buffer
 // loads made hipcc's host pass drop the kernel's launch stub.
-template <bool GATED, int NTT>
+template <bool GATED, int OUT_COLS, int NTT>
 __device__ __forceinline__ void thin_issue(f16* lds, __amdgpu_buffer_rsrc_t rx, __amdgpu_buffer_rsrc_t rw,
                                            __amdgpu_buffer_rsrc_t rw2, const unsigned* off, int wv,
                                            int ks, int buf) {
-    using C = Thin<GATED, NTT>;
+    using C = Thin<GATED, OUT_COLS, NTT>;
     static_assert((C::TW * kRowChunks) % kThinThreads == 0 && (C::OUT * kRowChunks) % kThinThreads == 0,
                   "the rows of load j lie in one operand for every wave");
     const unsigned soff = static_cast<unsigned>(ks) * kBK * 2u;
@@ -451,10 +452,10 @@ __device__ __forceinline__ void thin_issue(f16* lds, __amdgpu_buffer_rsrc_t rx, 
 
 // One thin tile: expert e's tail rows [row0, row_end) (tail = their count)
 // times output columns [col0, col0 + OUT).
-template <bool GATED, int NTT>
+template <bool GATED, int OUT_COLS, int NTT>
 __device__ __forceinline__ void thin_tile(const GemmArgs& a, f16* lds, int e, int row0, int row_end,
                                           int tail, int col0, int wv, int lane) {
-    using C = Thin<GATED, NTT>;
+    using C = Thin<GATED, OUT_COLS, NTT>;
     constexpr int NW = GATED ? 2 : 1;            // weight row tiles per wave
     constexpr int NT = C::NT;
     const int ct = wv % C::CT;                   // this wave's column tile
@@ -507,7 +508,7 @@ __device__ __forceinline__ void thin_tile(const GemmArgs& a, f16* lds, int e, in
     // (in bounds, never read as a stage), so every step issues one stage.
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s)
-        thin_issue<GATED, NTT>(lds, rx, rw, rw2, off, wv, stage(min(s, nk - 1)), s);
+        thin_issue<GATED, OUT_COLS, NTT>(lds, rx, rw, rw2, off, wv, stage(min(s, nk - 1)), s);
     for (int kt = 0; kt < nk; ++kt) {
         wait_vm<(NS - 2) * C::L>();   // this wave's loads of stage kt landed
         // Everyone's, and everyone is done with stage kt - 1. The empty asm
@@ -517,7 +518,7 @@ __device__ __forceinline__ void thin_tile(const GemmArgs& a, f16* lds, int e, in
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        thin_issue<GATED, NTT>(lds, rx, rw, rw2, off, wv, stage(min(kt + NS - 1, nk - 1)),
+        thin_issue<GATED, OUT_COLS, NTT>(lds, rx, rw, rw2, off, wv, stage(min(kt + NS - 1, nk - 1)),
                                (kt + NS - 1) % NS);   // into step kt - 1's buffer
         const f16* st = lds + static_cast<size_t>(kt % NS) * C::SH;
 #pragma unroll
@@ -568,9 +569,8 @@ __device__ __forceinline__ void thin_tile(const GemmArgs& a, f16* lds, int e, in
     }
 }
 
-template <bool GATED>
-__global__ __launch_bounds__(kThinThreads) void moe_expert_thin_kernel(const GemmArgs a) {
-    extern __shared__ __align__(16) f16 lds[];
+template <bool GATED, int OUT>
+__device__ __forceinline__ void thin_group(const GemmArgs& a, f16* lds) {
     const int e = blockIdx.y;
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -580,11 +580,24 @@ __global__ __launch_bounds__(kThinThreads) void moe_expert_thin_kernel(const Gem
     const int row0 = a.offsets[e] + (count - tail);
     const int row_end = min(a.offsets[e + 1], a.m_total);
     if (row0 < 0 || row0 >= row_end) return;
-    const int col0 = blockIdx.x * thin_out<GATED>();   // the grid covers n / OUT column tiles
+    const int col0 = blockIdx.x * OUT;   // the grid covers n / OUT column tiles
     // Uniform over the workgroup: the tile shape for this tail.
-    if (tail <= 32) thin_tile<GATED, 1>(a, lds, e, row0, row_end, tail, col0, wv, lane);
-    else if (tail <= 64) thin_tile<GATED, 2>(a, lds, e, row0, row_end, tail, col0, wv, lane);
-    else thin_tile<GATED, 4>(a, lds, e, row0, row_end, tail, col0, wv, lane);
+    if (tail <= 32) thin_tile<GATED, OUT, 1>(a, lds, e, row0, row_end, tail, col0, wv, lane);
+    else if (tail <= 64) thin_tile<GATED, OUT, 2>(a, lds, e, row0, row_end, tail, col0, wv, lane);
+    else thin_tile<GATED, OUT, 4>(a, lds, e, row0, row_end, tail, col0, wv, lane);
+}
+
+template <bool GATED>
+__global__ __launch_bounds__(kThinThreads) void moe_expert_thin_kernel(const GemmArgs a) {
+    extern __shared__ __align__(16) f16 lds[];
+    thin_group<GATED, thin_out<GATED>()>(a, lds);
+}
+
+// Plain, with OUT = 64 or 32 columns per workgroup (thin_columns below).
+template <int OUT>
+__global__ __launch_bounds__(kThinThreads) void moe_expert_thin_narrow_kernel(const GemmArgs a) {
+    extern __shared__ __align__(16) f16 lds[];
+    thin_group<false, OUT>(a, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -682,6 +695,48 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const CombineArgs a) {
     }
 }
 
+using ThinKernel = void (*)(GemmArgs);
+
+// Output columns per workgroup of a plain thin launch: the narrowest tile
+// whose grid still has at most one workgroup per CU, counting one expert per
+// row at most; 128 otherwise. A workgroup holds all of a CU's LDS and a CU
+// streams about 30 GB/s of weights, so with one token of top-2 and n 4096,
+// 64 workgroups of 128 columns left the other 192 CUs idle. Past one
+// workgroup per CU the narrower tile only re-reads more of the tail.
+// Measured (us per MoE layer, 128 / 64 / 32 columns): Mixtral's 8 x 4096 x
+// 14336 top-2, 1 token 163 / 144-155 / 139-160, 2 tokens 222 / 202-210 / 241,
+// 3 tokens 280 / 293 / 323, 64 tokens 447 / 447 / 526; 16 x 2048 x 4096 top-2,
+// 1 token 52 / 47.5 / 46.1, 4 tokens 81 / 73 / 86.5, 16 tokens 129 / 133 /
+// 157; one expert of 4096 x 14336, 20 tokens 131 / 108 / 102, 128 tokens 206 /
+// 164 / 143. Batches of 256 rows per expert or more, of which half the experts
+// have a tail, gained 1% at 64 columns or lost 2-4%. Gated
+// tiles of 32 columns instead of 64 gained only where one token met 16 such
+// experts (46.3 -> 44.2) and lost 10-20% elsewhere.
+constexpr long long kThinCUs = 256;  // MI355X
+
+int thin_columns(const GemmArgs& g) {
+    const long long experts = std::min(g.E, g.m_total);
+    for (int out : {32, 64}) {
+        if (g.n / out * experts <= kThinCUs) return out;
+    }
+    return thin_out<false>();
+}
+
+// The thin kernel's launch: a column tile per workgroup and an expert per row
+// of the grid; workgroups of experts without a short tail exit at once.
+hipError_t launch_thin(const GemmArgs& g, bool gated, hipStream_t stream) {
+    const int out = gated ? thin_out<true>() : thin_columns(g);
+    const ThinKernel fn = gated        ? moe_expert_thin_kernel<true>
+                          : out == 128 ? moe_expert_thin_kernel<false>
+                          : out == 64  ? moe_expert_thin_narrow_kernel<64>
+                                       : moe_expert_thin_narrow_kernel<32>;
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, kThinLds);
+    if (err != hipSuccess) return err;
+    return launch(fn, dim3(static_cast<unsigned>(g.n / out), static_cast<unsigned>(g.E)), dim3(kThinThreads),
+                  static_cast<size_t>(kThinLds), stream, g);
+}
+
 }  // namespace
 }  // namespace swiftllm
 
@@ -758,17 +813,8 @@ int swiftllm_hip_moe_expert_gemm(const void* a, const void* w, const void* w2,
         if (err != hipSuccess) return launched(err, who);
     }
     // The experts' short tails (at most kThinRows rows), which the main grid
-    // leaves out; workgroups of experts without one exit at once.
-    const dim3 thin(static_cast<unsigned>(n / (gated ? thin_out<true>() : thin_out<false>())),
-                    static_cast<unsigned>(num_experts));
-    const size_t tl = kThinLds;
-    const void* tf = gated ? reinterpret_cast<const void*>(moe_expert_thin_kernel<true>)
-                           : reinterpret_cast<const void*>(moe_expert_thin_kernel<false>);
-    err = hipFuncSetAttribute(tf, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(tl));
-    if (err != hipSuccess) return launched(err, who);
-    err = gated ? launch(moe_expert_thin_kernel<true>, thin, dim3(kThinThreads), tl, stream, g)
-                : launch(moe_expert_thin_kernel<false>, thin, dim3(kThinThreads), tl, stream, g);
-    return launched(err, who);
+    // leaves out.
+    return launched(launch_thin(g, gated, stream), who);
 }
 
 int swiftllm_hip_moe_combine(const void* y, const float* weights, const int32_t* inverse,

@@ -35,9 +35,9 @@ HIPCC = "/opt/rocm/bin/hipcc"
 THIN_LDS = 160 * 1024
 
 
-def thin_shape(gated, ntt):
-    """(loads per lane per stage L, ring stages NS) of a thin tile."""
-    out = 64 if gated else 128
+def thin_shape(gated, ntt, out=None):
+    """(loads per lane per stage L, ring stages NS) of a thin tile of `out` columns."""
+    out = out or (64 if gated else 128)
     tw = 2 * out if gated else out        # weight rows per stage
     rows = tw + 32 * ntt                  # plus the tail rows
     loads = rows * 8 // 256               # 16-byte chunks over 256 lanes
@@ -80,14 +80,14 @@ def main_wait_errors(body, n=8):
     return found, errs
 
 
-def thin_wait_errors(body, gated):
+def thin_wait_errors(body, gated, out=None):
     """Where a vmcnt(W > 0) wait of the thin kernel does not see exactly
     NS - 1 stages of direct-to-LDS loads in flight (so that it retires
     exactly the oldest stage) for one of the tile shapes. Returns (the
     (NTT, wait line) pairs matched, error strings)."""
     want = {}
     for ntt in (1, 2, 4):
-        L, NS = thin_shape(gated, ntt)
+        L, NS = thin_shape(gated, ntt, out)
         want.setdefault((NS - 2) * L, []).append((ntt, (NS - 1) * L))
     w = av.walk(body)
     matched, errs = set(), []
@@ -118,6 +118,15 @@ def test_main_kernel_wait_leaves_only_the_new_stage(asm, gated):
 @pytest.mark.parametrize("gated", [False, True])
 def test_thin_kernel_waits_retire_exactly_one_stage(asm, gated):
     matched, errs = thin_wait_errors(_body(asm, "moe_expert_thin_kernel", gated), gated)
+    assert not errs, errs
+    assert {ntt for ntt, _ in matched} == {1, 2, 4}, f"tile shapes with a checked wait: {matched}"
+
+
+@pytest.mark.parametrize("out", [64, 32])
+def test_narrow_thin_kernel_waits_retire_exactly_one_stage(asm, out):
+    """The plain thin kernel at 64 and 32 columns: shorter stages, longer rings."""
+    body = av.function_body(asm, av.mangled("moe_expert_thin_narrow_kernel", f"Li{out}E", "GemmArgs"))
+    matched, errs = thin_wait_errors(body, False, out)
     assert not errs, errs
     assert {ntt for ntt, _ in matched} == {1, 2, 4}, f"tile shapes with a checked wait: {matched}"
 

@@ -73,6 +73,34 @@ def test_expert_gemm_thin_tails(dev, gated, n, k):
            f"thin tails gated={gated} n={n} k={k}")
 
 
+@pytest.mark.parametrize("counts,n,k", [
+    ((0, 1, 0, 0, 0, 1, 0, 0), 4096, 64),     # 32 columns: 256 workgroups at most
+    ((1, 0, 0, 2, 0, 0, 0, 0), 4096, 64),     # 64 columns from here
+    ((0, 0, 4, 0, 0, 0, 0, 0), 4096, 64),     # 256 workgroups of 64 columns
+    ((1, 1, 1, 0, 0, 1, 0, 1), 4096, 64),     # 128 columns from here
+    ((32, 33), 256, 1280),                    # 20 stages, the ring of a one-tile tail
+    ((64, 65), 256, 1344),                    # 21
+    ((128, 129), 512, 832),
+    ((257, 100), 2048, 192),                  # 32 columns beside whole tiles
+    ((33, 1, 128, 5), 2048, 576),             # 64 columns, every tail shape
+])
+def test_expert_gemm_thin_columns(dev, counts, n, k):
+    """Plain thin tiles of 32, 64 and 128 columns around the lines of the rule
+    that chooses them, with k walks shorter than, as long as and longer than
+    the rings, and tails of one to four tiles."""
+    rng = np.random.default_rng(n + k + len(counts))
+    offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    a = (rng.standard_normal((int(offs[-1]), k)) * 0.5).astype(np.float16)
+    w = (rng.standard_normal((len(counts), n, k)) / np.sqrt(k)).astype(np.float16)
+    c = DeviceArray((int(offs[-1]), n), np.float16)
+    c.fill_byte(0xFF)
+    moe.moe_expert_gemm(DeviceArray.from_numpy(a), DeviceArray.from_numpy(w), None,
+                        DeviceArray.from_numpy(offs), c)
+    synchronize()
+    _close(c.numpy().astype(np.float64), oracle.moe_expert_gemm(a, w, None, offs),
+           f"thin columns {counts} n={n} k={k}")
+
+
 @pytest.mark.parametrize("gated", [False, True])
 def test_expert_gemm_many_experts(dev, gated):
     """160 experts: the main kernel's per-expert tile table is a wave scan in
