@@ -35,7 +35,8 @@
 // with ordinary (cached) loads: every query group of a sequence re-reads them.
 //
 // That kernel serves negative and zero scales, caches that are not 16-byte
-// aligned and batches of more than 1024 prompts; the usual call takes
+// aligned, batches of more than 1024 prompts and batches of prompts of a few
+// tokens; the usual call takes
 // paged_prefill_shared_kernel (below), whose waves share their stages.
 
 #include <algorithm>
@@ -527,7 +528,7 @@ void paged_prefill_kernel(const PrefillArgs a) {
 // (us per call, per-wave tiles -> this kernel): 8 x 2048 545 -> 443, 1 x 8192
 // 887 -> 734, 1 x 2048 82 -> 66, 24 prompts of 1-2457 tokens 241 -> 190, 64
 // of 16-200 60.8 -> 41.2, 4 x 1000-3000 of 16/16 heads 217 -> 157, 8 x 2048
-// of 8/8 heads x 64 101 -> 66, 1 x 17 7.0 -> 7.1. Of that, tiles longest first
+// of 8/8 heads x 64 101 -> 66. Of that, tiles longest first
 // against sequence by sequence: 208 -> 196 (24 prompts), 190 -> 165 (16/16
 // heads), 88 -> 70 (x 64); whole-row outputs 54 -> 43 (64 short prompts).
 // Loading the next tile's first stages and Q during a tile's last stage
@@ -537,6 +538,19 @@ constexpr int kSharedMaxSeqs = 1024;  // sequences in the LDS tile table
 constexpr long long kSharedCUs = 256;  // MI355X; any grid is correct, this one is resident at once
 template <int D>
 constexpr int kSharedPerCU = D == 128 ? 2 : 3;  // workgroups per CU, waves per SIMD
+
+// Query rows (tokens x heads of a kv head) of the longest prompt up to which
+// the per-wave kernel is the faster one: such a prompt is one short walk, and
+// finding its tile, the stage's barriers and the pass through LDS cost more
+// than they save. Measured (us per call, per-wave / shared): 1 prompt of 8/8
+// heads x 64 of 31 tokens 4.5 / 5.2, 94 tokens 6.1 / 6.7, 126 7.0 / 6.7; 16 of
+// up to 88 tokens 6.3 / 6.8, up to 124 7.4 / 7.0; 32/8 heads x 128, 4 of up to
+// 16 tokens 6.1 / 7.0, 23 tokens 7.0 / 7.0, 31 tokens 8.1 / 7.1; 64/8 x 128, 8
+// tokens 6.1 / 6.9, 11 6.8 / 6.9, 16 8.0 / 7.0. With more tiles than the grid
+// holds the line is lower: 64 prompts of 16/16 heads x 128 of up to 32 tokens
+// 11.3 / 13.1, 48 tokens 14.8 / 14.2.
+constexpr long long kBriefRows = 96;
+constexpr long long kBriefRowsMany = 32;
 
 typedef float f16x __attribute__((ext_vector_type(16)));
 
@@ -1061,7 +1075,9 @@ int prefill(const char* who, void* out, const void* q, const void* kc, const voi
     const int wide_heads = a.Hkv * ((a.G + 31) / 32);
     const long long wide_per = static_cast<long long>(kPrefillWaves) * (32 / wide_gw);
     const long long items = S * wide_heads * ((max_len + wide_per - 1) / wide_per);
-    if (fold && S <= kSharedMaxSeqs && items < (1LL << 30) && aligned(kc, 16) && aligned(vc, 16)) {
+    const long long resident = kSharedCUs * (D == 128 ? kSharedPerCU<128> : kSharedPerCU<64>);
+    const bool brief = max_len * a.G <= (items <= resident ? kBriefRows : kBriefRowsMany);
+    if (fold && !brief && S <= kSharedMaxSeqs && items < (1LL << 30) && aligned(kc, 16) && aligned(vc, 16)) {
         a.nhc = (a.G + 31) / 32;
         a.gw = wide_gw;
         a.tpw = 32 / wide_gw;
@@ -1070,7 +1086,7 @@ int prefill(const char* who, void* out, const void* q, const void* kc, const voi
         a.xcds = heads % 8 == 0 ? 8 : 1;
         a.q16 = aligned(q, 16);
         a.out16 = aligned(out, 16);
-        const long long wgs = std::min<long long>((items + 7) / 8 * 8, kSharedCUs * (D == 128 ? kSharedPerCU<128> : kSharedPerCU<64>));
+        const long long wgs = std::min<long long>((items + 7) / 8 * 8, resident);
         return launched(launch(D == 128 ? paged_prefill_shared_kernel<128> : paged_prefill_shared_kernel<64>,
                                dim3(static_cast<unsigned>(wgs)), block, 0, stream, a),
                         who);

@@ -258,7 +258,7 @@ def test_prefill_first_block_out_of_pool(dev, H, Hkv, D):
     that see only that block attend to no key and come out as zeros, beside
     rows of the same wave that see the next block. The others attend to the
     keys from position 16 on, as a prompt that starts there would."""
-    L = 90
+    L = 120
     w = workloads.prefill_config((L, 33), H, Hkv, D, seed=31 + D)
     w.slot_mapping[:16] = -1
     out = _run(w)
@@ -266,3 +266,15 @@ def test_prefill_first_block_out_of_pool(dev, H, Hkv, D):
     ref = oracle.prefill_numpy(w.q[16:], w.key_cache, w.value_cache, w.slot_mapping[16:],
                                np.array([L - 16, 33]), w.scale)
     assert_attention_close(out[16:], ref, f"prefill first block out H{H} Hkv{Hkv} D{D}")
+
+
+@pytest.mark.parametrize("H,Hkv,D,lens", [
+    (8, 8, 64, (96, 5)), (8, 8, 64, (97, 5)),             # rows at and past the line, few tiles
+    (32, 8, 128, (24, 0, 1)), (32, 8, 128, (25, 0, 1)),
+    (40, 1, 128, (2, 1)), (40, 1, 128, (3, 1)),
+    (16, 16, 128, (32, 1) * 20), (16, 16, 128, (33, 1) * 20),   # more tiles than the grid holds
+])
+def test_prefill_prompts_of_a_few_tokens(dev, H, Hkv, D, lens):
+    """The line between the per-wave and the shared-stage kernel."""
+    w = workloads.prefill_config(lens, H, Hkv, D, seed=H + max(lens))
+    assert_attention_close(_run(w), _ref(w), f"prefill H{H} Hkv{Hkv} D{D} up to {max(lens)}")
