@@ -502,7 +502,8 @@ constexpr int kLdsPad = 512;           // room for one more column (E >= 8)
 // lines they hold are written back at the kernel's end instead. Measured (us
 // per call, 8 experts, top-2, nontemporal / plain): 67 MB of rows 20.5 / 19.3,
 // 47.5 MB 15.3 / 15.3, 32.8 MB 11.8 / 12.9, 16.4 MB 8.6 / 9.7; 64 experts,
-// top-6, 100 MB 31.1 / 29.7.
+// top-6, 100 MB 31.1 / 29.7. That is with the same rows written by every call;
+// with eight row sets of 67 MB in turn both take 21.3.
 constexpr size_t kNontemporalRows = 48u << 20;
 
 struct PermuteArgs {
