@@ -193,6 +193,13 @@ __device__ __forceinline__ void mask_tail(int nv, int kg, h4 (&kA)[D / 16], h4 (
     }
 }
 
+// The factor a row's sums take when its maximum moves from m to m_new. A row
+// that has seen no key yet (its blocks are outside the pool) may sit in a wave
+// beside one that has: it keeps its zeros, which -inf - -inf would make NaN.
+__device__ __forceinline__ float rescale(float m, float m_new) {
+    return (m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+}
+
 // Steps 3 + 4 for one group of 16 query rows, from the S^T accumulator sc.
 // Lane (r, kg) holds S^T[t = 4kg + i][g = r].
 // PV32 runs PV on the 16x16x32 form: k = 8q + i is token 4q + i of the hi
@@ -226,7 +233,7 @@ __device__ __forceinline__ void softmax_pv(WaveState<D>& st, f4 sc, int lim, int
     if constexpr (FOLD) bm *= scale_log2;
     if (__any(bm > (LAZY ? st.m + kLazyMargin : st.m))) {
         const float m_new = fmaxf(st.m, bm);
-        const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
+        const float alpha = rescale(st.m, m_new);
 #pragma unroll
         for (int J = 0; J < NJ; ++J) st.acc[J] *= alpha;
         st.l *= alpha;

@@ -141,7 +141,7 @@ __device__ __forceinline__ void softmax_pv_pair(WaveState<D>& st, f4 s0, f4 s1, 
     if constexpr (FOLD) bm *= scale_log2;
     if (__any(bm > st.m + kLazyMargin)) {
         const float m_new = fmaxf(st.m, bm);
-        const float alpha = __builtin_amdgcn_exp2f(st.m - m_new);
+        const float alpha = rescale(st.m, m_new);
 #pragma unroll
         for (int J = 0; J < NJ; ++J) st.acc[J] *= alpha;
         st.l *= alpha;
@@ -898,9 +898,7 @@ void paged_prefill_shared_kernel(const PrefillArgs a) {
             }
             if (__any(bm > m + kLazyMargin)) {
                 const float m_new = fmaxf(m, bm);
-                // A row that has seen no key yet (its blocks are outside the
-                // pool) keeps its zeros: -inf - -inf would make them NaN.
-                const float alpha = (m_new == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+                const float alpha = rescale(m, m_new);
 #pragma unroll
                 for (int i = 0; i < ND; ++i) acc[i] *= alpha;
                 l *= alpha;

@@ -278,3 +278,38 @@ def test_prefill_prompts_of_a_few_tokens(dev, H, Hkv, D, lens):
     """The line between the per-wave and the shared-stage kernel."""
     w = workloads.prefill_config(lens, H, Hkv, D, seed=H + max(lens))
     assert_attention_close(_run(w), _ref(w), f"prefill H{H} Hkv{Hkv} D{D} up to {max(lens)}")
+
+
+def _run_key_offset(w, key_offset):
+    """_run with the key cache key_offset bytes past a 16-byte boundary."""
+    T, H, D = w.q.shape
+    kc = DeviceArray((w.key_cache.size + 8,), np.float16)
+    kc.upload_at(key_offset, w.key_cache)
+    out = DeviceArray((T, H, D), np.float16)
+    out.fill_byte(0xFF)
+    q, vc = DeviceArray.from_numpy(w.q), DeviceArray.from_numpy(w.value_cache)
+    sm, ctx = DeviceArray.from_numpy(w.slot_mapping), DeviceArray.from_numpy(w.context_lens)
+    pa.launch_paged_prefill(out, q, kc.ptr + key_offset, vc, sm, ctx, w.scale, len(w.context_lens), H,
+                            w.key_cache.shape[1], D, 16, int(w.context_lens.max()),
+                            num_blocks=w.key_cache.shape[0])
+    synchronize()
+    return out.numpy()
+
+
+@pytest.mark.parametrize("H,Hkv,D,L,sign,key_offset", [
+    (6, 2, 64, 30, 1, 0), (6, 2, 128, 30, 1, 0), (10, 2, 128, 19, 1, 0),  # prompts of a few tokens
+    (6, 2, 64, 120, -1, 0), (10, 2, 128, 120, -1, 0),                     # a negative scale
+    (6, 2, 128, 120, 1, 8), (10, 2, 64, 120, 1, 8), (10, 2, 64, 120, -1, 8),  # K through registers
+])
+def test_prefill_first_block_out_of_pool_per_wave(dev, H, Hkv, D, L, sign, key_offset):
+    """The same in the per-wave kernel, on each of its calls: with 3 or 5 heads
+    to a kv head a group of 16 query rows holds tokens of the first block
+    (which see no key) and of the second, whose maxima rescale the group."""
+    w = workloads.prefill_config((L, 13), H, Hkv, D, seed=37 + D + L)
+    w = dataclasses.replace(w, scale=sign * w.scale)
+    w.slot_mapping[:16] = -1
+    out = _run_key_offset(w, key_offset)
+    assert np.array_equal(out[:16].view(np.uint16), np.zeros((16, H, D), np.uint16))
+    ref = oracle.prefill_numpy(w.q[16:], w.key_cache, w.value_cache, w.slot_mapping[16:],
+                               np.array([L - 16, 13]), w.scale)
+    assert_attention_close(out[16:], ref, f"prefill first block out H{H} Hkv{Hkv} D{D} L{L}")
