@@ -247,7 +247,10 @@ int swiftllm_hip_reshape_and_cache(const void* key, const void* value,
  * [start_s, start_s + context_lens[s]), start_s the sum of the lengths
  * before it. Token i of s attends to tokens j <= i of s, whose K/V sit in
  * the cache at slot_mapping[start_s + j]; the slots of a sequence must walk
- * its block table from position 0 (table[p / 16] * 16 + p % 16).
+ * its block table from position 0 (table[p / 16] * 16 + p % 16). A value that
+ * is not finite also makes NaN of earlier tokens that one wave (32 query
+ * rows) serves together with a token of its 16-token block or a later one;
+ * a key that is not finite does not.
  * params->max_context_len bounds every context_lens[s]; above 2^24 tokens it
  * can return SWIFTLLM_ERR_NOT_SUPPORTED (grid size). */
 int swiftllm_hip_paged_attention_prefill(

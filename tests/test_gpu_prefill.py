@@ -313,3 +313,26 @@ def test_prefill_first_block_out_of_pool_per_wave(dev, H, Hkv, D, L, sign, key_o
     ref = oracle.prefill_numpy(w.q[16:], w.key_cache, w.value_cache, w.slot_mapping[16:],
                                np.array([L - 16, 13]), w.scale)
     assert_attention_close(out[16:], ref, f"prefill first block out H{H} Hkv{Hkv} D{D} L{L}")
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(8, 8, 64), (8, 8, 128), (8, 4, 64), (6, 2, 128), (32, 8, 128),
+                                     (64, 8, 64)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_prefill_non_finite_value_stays_near_its_token(dev, H, Hkv, D, bad):
+    """A value that is not finite reaches the tokens that attend to it and, as
+    0 times it is NaN, earlier ones of the same wave: at most 32 tokens that
+    end in its block or later. Tokens before 80 share no wave with one past 95
+    (32 or 16 tokens a wave, aligned, or at most 10), so token 100 of a
+    300-token prompt leaves them as they are, whatever a workgroup spans."""
+    w = workloads.prefill_config((300,), H, Hkv, D, seed=41 + D)
+    ref = _ref(w)
+    b, o = w.slot_mapping[100] // 16, w.slot_mapping[100] % 16
+    w.value_cache[b, :, :, o] = bad
+    for sign in (1, -1):
+        v = dataclasses.replace(w, scale=sign * w.scale)
+        if sign < 0:
+            ref = oracle.prefill_numpy(w.q[:96], w.key_cache, w.value_cache, w.slot_mapping[:96],
+                                       np.array([96]), v.scale)
+        out = _run(v)
+        assert_attention_close(out[:80], ref[:80], f"prefill, {bad} in V at 100, H{H} Hkv{Hkv} D{D} {sign}")
+        assert not np.isfinite(out[100:].astype(np.float64)).any(), "every later token attends to it"
