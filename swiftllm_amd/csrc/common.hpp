@@ -138,6 +138,11 @@ __device__ __forceinline__ int wave_inclusive_scan(int x) {
     return dpp_scan(x, 0, [](int a, int b) { return a + b; });
 }
 
+// The maximum of x >= 0 over the wave.
+__device__ __forceinline__ int wave_max(int x) {
+    return __builtin_amdgcn_readlane(dpp_scan(x, 0, [](int a, int b) { return max(a, b); }), 63);
+}
+
 // The sum of x over the wave.
 __device__ __forceinline__ int wave_total(int x) {
     return __builtin_amdgcn_readlane(wave_inclusive_scan(x), 63);

@@ -547,10 +547,15 @@ constexpr int kSharedPerCU = D == 128 ? 2 : 3;  // workgroups per CU, waves per 
 // up to 88 tokens 6.3 / 6.8, up to 124 7.4 / 7.0; 32/8 heads x 128, 4 of up to
 // 16 tokens 6.1 / 7.0, 23 tokens 7.0 / 7.0, 31 tokens 8.1 / 7.1; 64/8 x 128, 8
 // tokens 6.1 / 6.9, 11 6.8 / 6.9, 16 8.0 / 7.0. With more tiles than the grid
-// holds the line is lower: 64 prompts of 16/16 heads x 128 of up to 32 tokens
-// 11.3 / 13.1, 48 tokens 14.8 / 14.2.
+// holds the line is lower, and where every head has its own kv head (a row is a
+// token there, and walks as many keys) it lies elsewhere for each head_dim.
+// Per-wave time over shared, 65 to 1000 prompts of equal lengths / of 1 up to
+// the same: 2 to 8 heads to a kv head, 64 rows 0.71-1.14 / 0.66-0.96, 96 rows
+// 0.96-1.43 / 0.79-1.17; 8/8 x 64, 96 rows 0.85-0.99 / 0.73-0.84, 128 rows
+// 0.94-1.21 / 0.84-0.96; 16/16 x 128, 32 rows 0.85-0.99 / 0.77-0.88, 64 rows
+// 0.98-1.13 / 0.90-1.10.
 constexpr long long kBriefRows = 96;
-constexpr long long kBriefRowsMany = 32;
+constexpr long long brief_rows_many(int G, int D) { return G > 1 ? 64 : D == 64 ? 96 : 32; }
 
 typedef float f16x __attribute__((ext_vector_type(16)));
 
@@ -645,6 +650,7 @@ struct TileTable {
     int S;
     int tiles;     // S <= 64: of sequence `lane`
     int start;
+    int top;       // tiles of the longest sequence
     __device__ __forceinline__ int tiles_of(int s0, int lane) const {
         if (S <= 64) return tiles;
         return s0 + lane < S ? lds->tiles[s0 + lane] : 0;
@@ -662,27 +668,35 @@ struct TileTable {
 
 __device__ __forceinline__ TileTable make_tiles(const int* ctx, int S, int per_wg, int max_tiles, TileLds* lds,
                                                 int* s_part) {
-    TileTable t{lds, S, 0, 0};
+    TileTable t{lds, S, 0, 0, 0};
     const int lane = threadIdx.x & 63;
     if (S <= 64) {
         const int len = lane < S ? max(ctx[lane], 0) : 0;
         t.tiles = min((len + per_wg - 1) / per_wg, max_tiles);
         t.start = wave_inclusive_scan(len) - len;
+        t.top = wave_max(t.tiles);
         return t;
     }
     constexpr int kEach = kSharedMaxSeqs / (64 * kPrefillWaves);
     const int c0 = threadIdx.x * kEach;
     int len[kEach];
-    int sum = 0;
+    int sum = 0, most = 0;
 #pragma unroll
     for (int i = 0; i < kEach; ++i) {
         len[i] = c0 + i < S ? max(ctx[c0 + i], 0) : 0;
         sum += len[i];
+        most = max(most, len[i]);
     }
+    most = wave_max(most);
     const int incl = wave_inclusive_scan(sum);
     const int w = threadIdx.x >> 6;
-    if (lane == 63) s_part[w] = incl;
+    if (lane == 63) {
+        s_part[w] = incl;
+        s_part[kPrefillWaves + w] = most;
+    }
     __syncthreads();
+    for (int i = 0; i < kPrefillWaves; ++i) most = max(most, s_part[kPrefillWaves + i]);
+    t.top = min((most + per_wg - 1) / per_wg, max_tiles);
     int at = incl - sum;
     for (int i = 0; i < w; ++i) at += s_part[i];
 #pragma unroll
@@ -700,8 +714,8 @@ __device__ __forceinline__ TileTable make_tiles(const int* ctx, int S, int per_w
 // Entry e (below count(0)) of the list of (tile, sequence) pairs, highest tile
 // index (longest walk) first, sequences in order within one index. Every wave
 // works it out for itself.
-__device__ __forceinline__ void nth_tile(const TileTable& tt, int max_tiles, int e, int lane, int& tile, int& seq) {
-    int lo = 0, hi = max_tiles, below = 0;  // count(lo) > e >= count(hi) = below
+__device__ __forceinline__ void nth_tile(const TileTable& tt, int e, int lane, int& tile, int& seq) {
+    int lo = 0, hi = tt.top, below = 0;  // count(lo) > e >= count(hi) = below
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         const int n = tt.count(mid, lane);
@@ -733,7 +747,7 @@ void paged_prefill_shared_kernel(const PrefillArgs a) {
     constexpr int NJ = D / 16;   // 16-wide k steps of QK^T
     constexpr int ND = D / 32;   // 32-row pieces of the output
     using St = Stage<D>;
-    __shared__ int s_part[kPrefillWaves];
+    __shared__ int s_part[2 * kPrefillWaves];
     __shared__ TileLds s_tiles;
     __shared__ __align__(16) f16 s_k[2][St::kK];
     __shared__ __align__(16) f16 s_v[2][St::kV];
@@ -773,7 +787,7 @@ void paged_prefill_shared_kernel(const PrefillArgs a) {
     const unsigned item = item_of(round);
     const unsigned e = item / heads;
     int tile, s;
-    nth_tile(tt, a.groups, static_cast<int>(e), lane, tile, s);
+    nth_tile(tt, static_cast<int>(e), lane, tile, s);
     s = __builtin_amdgcn_readfirstlane(s);
     tile = __builtin_amdgcn_readfirstlane(tile);
     const int yy = static_cast<int>(x + a.xcds * (item - e * heads));
@@ -1085,7 +1099,7 @@ int prefill(const char* who, void* out, const void* q, const void* kc, const voi
     const long long wide_per = static_cast<long long>(kPrefillWaves) * (32 / wide_gw);
     const long long items = S * wide_heads * ((max_len + wide_per - 1) / wide_per);
     const long long resident = kSharedCUs * (D == 128 ? kSharedPerCU<128> : kSharedPerCU<64>);
-    const bool brief = max_len * a.G <= (items <= resident ? kBriefRows : kBriefRowsMany);
+    const bool brief = max_len * a.G <= (items <= resident ? kBriefRows : brief_rows_many(a.G, static_cast<int>(D)));
     if (fold && !brief && S <= kSharedMaxSeqs && items < (1LL << 30) && aligned(kc, 16) && aligned(vc, 16)) {
         a.nhc = (a.G + 31) / 32;
         a.gw = wide_gw;

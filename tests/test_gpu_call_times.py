@@ -1,0 +1,52 @@
+"""Calls whose route is chosen by their sizes, against another route to the
+same result: the chosen one must not cost a multiple of the other. Times are
+the best of several replays of a graph of equal calls, so the host's part is
+not in them, and the margins are far above what two runs differ by."""
+
+import numpy as np
+import pytest
+
+from swiftllm_amd import paged_attention as pa
+from swiftllm_amd._hip import DeviceArray, Event, Graph, Stream
+
+pytestmark = pytest.mark.gpu
+
+
+def best_us(call, calls=20, replays=8):
+    """Microseconds per call(stream)."""
+    stream = Stream()
+    call(stream)  # code objects are loaded before the capture
+    stream.synchronize()
+    graph = Graph(stream, lambda: [call(stream) for _ in range(calls)])
+    best = float("inf")
+    for _ in range(replays):
+        a, b = Event(), Event()
+        a.record(stream)
+        graph.launch(stream)
+        b.record(stream)
+        b.synchronize()
+        best = min(best, a.elapsed_ms(b) * 1e3 / calls)
+    return best
+
+
+@pytest.mark.parametrize("S,L,H,Hkv,D", [(1000, 64, 8, 8, 64), (300, 16, 32, 8, 128)])
+def test_many_short_prompts(dev, S, L, H, Hkv, D):
+    """A positive scale may take the kernel with shared stages, a negative one
+    takes the per-wave kernel: on many prompts of a few tokens a positive one
+    costs no more (at most 64 tokens each, 8/8 x 64: 60 us against 46 where
+    such calls shared their stages)."""
+    rng = np.random.default_rng(S + L)
+    lens = rng.integers(1, L + 1, size=S).astype(np.int32)
+    lens[0] = L
+    nb = (lens + 15) // 16
+    first = np.cumsum(nb) - nb
+    slots = np.concatenate([16 * f + np.arange(n) for f, n in zip(first, lens)]).astype(np.int32)
+    T, NB = int(lens.sum()), int(nb.sum())
+    def arr(*shape):
+        return DeviceArray.from_numpy((rng.standard_normal(shape) * 0.5).astype(np.float16))
+    q, kc, vc = arr(T, H, D), arr(NB, Hkv, D, 16), arr(NB, Hkv, D, 16)
+    sm, ctx, out = DeviceArray.from_numpy(slots), DeviceArray.from_numpy(lens), DeviceArray((T, H, D), np.float16)
+    us = [best_us(lambda stream: pa.launch_paged_prefill(out, q, kc, vc, sm, ctx, sign / np.sqrt(D), S, H, Hkv, D,
+                                                         16, L, num_blocks=NB, stream=stream))
+          for sign in (1, -1)]
+    assert us[0] < 1.12 * us[1], f"{us[0]:.1f} us, per wave {us[1]:.1f} us"
