@@ -234,7 +234,14 @@ __global__ __launch_bounds__(256) void reshape_and_cache_runs_kernel(const Cache
 // windows of 4 and 6.4 us in windows of 16 (5.3 us token by token), 256 take
 // 9.2 and 10.0 (9.5). Past it windows of 16 leave fewer workgroups that find
 // no head: 1024 lone tokens take 29.0 us with them (29.6 token by token).
+// A layer of few rows leaves few workgroups at any window, and short runs pay
+// for it, one after the other in a window: up to kSmallPieces tokens times
+// slices of 256 rows it keeps windows of 4. Measured in runs of 2 tokens,
+// windows of 4 / 16 (token by token): 513 tokens of 2 x 128 5.4 / 9.8 (6.2),
+// of 1 x 128 4.0 / 6.8 (4.7), 1024 of 2 x 128 6.8 / 9.9 (9.1), 2048 12.5 / 12.2
+// (15.6); in one run 1024 of 2 x 128 3.8 / 4.0, of 8 x 64 4.4 / 3.9.
 constexpr int kSmallTokens = 512;
+constexpr long long kSmallPieces = 1024;
 
 int reshape_and_cache(const void* key, const void* value, void* key_cache, void* value_cache,
                       const int* slot_mapping, int num_tokens, int num_kv_heads, int head_dim,
@@ -269,7 +276,7 @@ int reshape_and_cache(const void* key, const void* value, void* key_cache, void*
     a.BS = block_size;
     const long long n = static_cast<long long>(num_kv_heads) * head_dim;
     const long long slices = (n + kWinRows - 1) / kWinRows;
-    const int W = num_tokens <= kSmallTokens ? 4 : 16;
+    const int W = num_tokens <= kSmallTokens || num_tokens * slices <= kSmallPieces ? 4 : 16;
     const long long windows = (static_cast<long long>(num_tokens) + W - 1) / W;
     if (block_size == kBlockTokens && n % 16 == 0 && windows < (1 << 24) && slices <= 65535 &&
         aligned(key, 16) && aligned(value, 16) && aligned(key_cache, 8) && aligned(value_cache, 8)) {
