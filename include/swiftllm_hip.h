@@ -110,13 +110,15 @@ void launch_reshape_and_cache(void* key, void* value, void* key_cache,
  * batch's lengths leave each workgroup of the GPU. Batches of few sequences
  * (at most two per team of workgroups, where the workspace has the room) are
  * cut into equal ranges of blocks instead, one per team, whatever the
- * partitions, and tables too short for a split to pay are attended in a
- * single pass; the size query's answer depends on the current device's
- * compute units.
+ * partitions, and tables too short for a split to pay (at most 96 blocks)
+ * are attended in a single pass; the size query's answer depends on the
+ * current device's compute units.
  * partition_size 0 selects balanced scheduling: the blocks of all sequences
- * are always split into equal ranges, one per team of waves for large
- * batches, so a ragged batch has no long tail; ranges that cut a sequence
- * leave fragments that a second kernel combines. Shapes it cannot take (more
+ * are split into equal ranges, one per team of waves for large batches, so
+ * a ragged batch has no long tail; ranges that cut a sequence leave
+ * fragments that a second kernel combines. Tables of at most 64 blocks (32
+ * for more than four sequences times kv heads per compute unit), whose
+ * longest context is no long tail, may run in a single pass. Shapes it cannot take (more
  * than 4096 sequences, or teams so wide that fewer than four fit in the
  * resident grid) fall back to partitions of 512 tokens; the workspace size
  * query covers both.

@@ -1359,13 +1359,24 @@ int decode_v1(void* out, const void* q, const void* kc, const void* vc, const in
 // pass reads at the same rate. Measured (us per call, single pass / teams,
 // all contexts of one length, 32/8 heads x 128): 1 sequence of 512 tokens 7.8
 // / 8.2, of 1024 11.4 / 9.1; 8 of 512 9.2 / 10.8, of 1024 14.9 / 12.8; 16 of
-// 1024 16.4 / 17.4, of 2048 29.3 / 27.2; 32 of 2048 41.6 / 46.8; 64 of
-// 64-1024 25.9 / 34.1; items: 128 of 200-400 28.8 / 31.0, 256 of 1-1024
-// lognormal 106 / 105.
-bool single_pass(const Shape& sh, int cus) {
+// 1024 16.4 / 17.4; 64 of 64-1024 25.9 / 34.1; items: 128 of 200-400 28.8 /
+// 31.0, 256 of 1-1024 lognormal 106 / 105.
+// The table says nothing of the other contexts, and one long context among
+// short ones is the single pass's worst: its whole chain runs on one workgroup
+// per kv head. So a table past 96 blocks is split whatever the batch, and past
+// 64 (32 with more than four items per CU) in balanced mode, whose ranges are
+// for such batches. All but one of 32 tokens (us per call, single pass / split):
+// 64 sequences, one of 1536 tokens 22 / 26 in 512-token items (12 by teams),
+// 2500 31.9 / 15.0; 96, one of 3500 43.6 / 19.1; balanced 48, one of 1280 17.0
+// / 11.5, of 2048 24.3 / 11.8; 256, one of 1024 20.9 / 15.3. Even contexts pay
+// for it above the line: 32 of 1536 tokens balanced 30.7 / 35.9, 64 of 128-2048
+// in 512-token partitions 49.5 / 55.8, 256 of 1024 balanced 157 / 185.
+bool single_pass(const Shape& sh, int partition_size, int cus) {
     if (sh.S > kPartMaxSeqs) return false;
+    const bool balanced = partition_size == 0;
     const long long items = static_cast<long long>(sh.S) * sh.Hkv * ((sh.H / sh.Hkv + 15) / 16);
-    return sh.MB <= (items <= 3LL * cus ? 32 + items / 4 : kSingleRoundBlocks);
+    if (items > 3LL * cus) return sh.MB <= (balanced && items > 4LL * cus ? 32 : 64);
+    return sh.MB <= std::min(32 + items / 4, balanced ? 64LL : 96LL);
 }
 
 // Split-K workspace: max logits and exp sums [S][H][MP] and partial outputs
@@ -1604,7 +1615,7 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
             return fail(SWIFTLLM_ERR_INVALID_PARAMETER, "%s: workspace of %zu bytes, %zu needed", who,
                         ws_bytes, need.total);
         }
-        if (single_pass(sh, device_cus())) {
+        if (single_pass(sh, partition_size, device_cus())) {
             return decode_v1(out, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
         }
         const TeamNeed team = team_need(sh, device_cus());
@@ -1625,7 +1636,7 @@ int decode_v2(void* out, void* ws, size_t ws_bytes, const void* q, const void* k
     }
     if ((rc = require_device()) != SWIFTLLM_OK) return rc;
     if (sh.S == 0) return ok();
-    if (single_pass(sh, device_cus())) {
+    if (single_pass(sh, partition_size, device_cus())) {
         return decode_v1(out, q, kc, vc, bt, ctx, scale, sh, num_blocks, stream, who);
     }
     const TeamNeed team = team_need(sh, device_cus());

@@ -69,3 +69,41 @@ def test_cache_write_of_short_runs(dev, Hkv, D):
                                                              D, 16, num_blocks=NB, stream=stream))
           for shift in (0, 4)]
     assert us[0] < 1.2 * us[1], f"{us[0]:.2f} us, token by token {us[1]:.2f} us"
+
+
+class _Decode:
+    """A decode batch whose contexts take random blocks of a small pool."""
+
+    def __init__(self, lens, H, Hkv, D, table_blocks):
+        rng = np.random.default_rng(len(lens))
+        self.lens = np.asarray(lens, np.int32)
+        S, NB = len(lens), 4096
+        self.shape = (S, H, Hkv, D, 16, table_blocks)
+        self.nb, self.scale = NB, 1.0 / np.sqrt(D)
+        fill = (rng.standard_normal((NB * Hkv * D * 16,)) * 0.5).astype(np.float16)
+        self.kc, self.vc = DeviceArray.from_numpy(fill), DeviceArray.from_numpy(fill[::-1].copy())
+        self.q = DeviceArray.from_numpy(rng.standard_normal((S, H, D)).astype(np.float16))
+        self.bt = DeviceArray.from_numpy(rng.integers(0, NB, (S, table_blocks)).astype(np.int32))
+        self.ctx = DeviceArray.from_numpy(self.lens)
+        self.out = DeviceArray((S, H, D), np.float16)
+
+    def v1(self, stream):
+        pa.paged_attention_v1(self.out, self.q, self.kc, self.vc, self.bt, self.ctx, self.scale, *self.shape,
+                              num_blocks=self.nb, stream=stream)
+
+    def v2(self, partition):
+        ws = pa.workspace(pa.paged_attention_v2_workspace_size(*self.shape, partition))
+        return lambda stream: pa.paged_attention_v2(self.out, ws, self.q, self.kc, self.vc, self.bt, self.ctx,
+                                                    self.scale, *self.shape, partition, num_blocks=self.nb,
+                                                    stream=stream)
+
+
+@pytest.mark.parametrize("S,long", [(64, 2500), (96, 3500)])
+@pytest.mark.parametrize("partition", [512, 0])
+def test_one_long_context_among_short_ones_is_split(dev, S, long, partition):
+    """All contexts of 32 tokens but one: a split call spreads the long one over
+    workgroups, where the single pass walks it in one per kv head (64 with one
+    of 2500 tokens 32 us and split 15, 96 with one of 3500 44 and 19)."""
+    d = _Decode([32] * (S - 1) + [long], 32, 8, 128, (long + 15) // 16)
+    split, single = best_us(d.v2(partition)), best_us(d.v1)
+    assert split < 0.75 * single, f"{split:.1f} us, single pass {single:.1f} us"
