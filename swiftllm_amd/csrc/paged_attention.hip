@@ -67,6 +67,7 @@ struct DecodeArgs {
     int MP;           // partitions per sequence in the workspace
     int S;            // sequences
     float share;      // split-K items: kItemShare of a resident workgroup, per block of the batch
+    bool single;      // the partition kernel runs a single-pass call
     int snake;        // > 0: single-pass item order in snake rounds of this many
 };
 
@@ -203,9 +204,10 @@ __host__ __device__ constexpr size_t part_list_lds_bytes(int S) {
 // workgroup take the item's blocks round-robin and merge through LDS; the
 // result is the output (single pass, or a sequence with one partition) or a
 // split-K partial. Every thread of the workgroup calls it with the same item.
+// `len`: the sequence's context length where the caller has it, else -1.
 template <int D, int NW>
 __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh, int hc,
-                                            int part, int part_blocks) {
+                                            int part, int part_blocks, int len = -1) {
     constexpr int NJ = D / 16;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -217,8 +219,8 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, int s, int kvh,
     const int gstride = min(16, a.G);  // LDS rows per wave
     const int h0 = kvh * a.G + g0;
 
-    int L = a.ctx[s];
-    L = max(L, 0);
+    int L = len;
+    if (len < 0) L = max(a.ctx[s], 0);
     const int nblk = min((L + kBlockTokens - 1) / kBlockTokens, a.MB);
     L = min(L, nblk * kBlockTokens);
     int nparts, jb0, jb1;
@@ -360,14 +362,49 @@ constexpr int kLptClasses = 16;
 // for itself, from the lengths alone.
 constexpr float kItemShare = 1.5f;
 
-__device__ __forceinline__ int item_blocks(const int* ctx, int S, int MB, int part_blocks, float share) {
-    int sum = 0;
+// Blocks of the batch's contexts, each counted as 2^18 (4M tokens) at most, so
+// that kPartMaxSeqs of them fit in an int; every wave works them out for itself.
+struct BatchBlocks {
+    int sum, longest;
+    int len;  // context length of sequence `s`
+};
+
+__device__ __forceinline__ BatchBlocks batch_blocks(const int* ctx, int S, int MB, int s) {
+    BatchBlocks b{0, 0, 0};
+    const int cap = min(MB, 1 << 18);
+#pragma unroll 4
     for (int i = threadIdx.x & 63; i < S; i += 64) {
-        // (2^18 blocks are 4M tokens: kPartMaxSeqs such contexts fit in an int)
-        sum += min(min((max(ctx[i], 0) + kBlockTokens - 1) / kBlockTokens, MB), 1 << 18);
+        const int len = max(ctx[i], 0);
+        const int n = min((len + kBlockTokens - 1) / kBlockTokens, cap);
+        b.sum += n;
+        b.longest = max(b.longest, n);
+        b.len = (i ^ s) < 64 ? len : b.len;  // lanes of s's group of 64
     }
-    const int most = static_cast<int>(fminf(static_cast<float>(wave_total(sum)) * share, 0x1p28f));
+    return BatchBlocks{wave_total(b.sum), wave_max(b.longest), __builtin_amdgcn_readlane(b.len, s & 63)};
+}
+
+__device__ __forceinline__ int item_blocks(const int* ctx, int S, int MB, int part_blocks, float share) {
+    const int sum = batch_blocks(ctx, S, MB, 0).sum;
+    const int most = static_cast<int>(fminf(static_cast<float>(sum) * share, 0x1p28f));
     return __builtin_amdgcn_readfirstlane(part_blocks * max(1, most / part_blocks));
+}
+
+// Whether a single-pass batch is run through the list (one item per sequence,
+// longest first) or in plain order. The table's width says nothing of the
+// contexts, so the kernel looks at them. Plain order ends later than the list
+// by the time its longest context still takes once the others are done, at
+// most its chain and at most the batch's time; the list costs every workgroup
+// its prologue, about 0.04 us per sequence. So: a longest context of some
+// length for the number of sequences, work enough before it, and well above the
+// mean. Measured (us per call, plain / list, tables 512 blocks wide): 256
+// lognormal contexts, 32/8 heads x 128, 227 / 198; 96, 16/16 x 128, 118 / 102;
+// 128 of 64-1024 tokens, 32/8 x 128, 54.5 / 52.6, 8/8 x 64 25.9 / 28.4; 256 of
+// 16-128 17.0 / 27.4, 8/8 x 64 9.3 / 17.5; 1024 of 16-128 63.6 / 102.5; 127 of
+// 32 beside one of 2500, 8/8 x 64, 19.9 / 21.9; 128 of 1024 80.0 / 82.1.
+template <int D>
+__device__ __forceinline__ bool list_pays(BatchBlocks b, int S, int HC) {
+    return b.longest * (D / 64) > 2 * (S / 4 + 16) && static_cast<float>(b.sum) * HC > 32.0f * S &&
+           2.0f * b.longest * S > 3.0f * b.sum;
 }
 
 template <int D, int NW>
@@ -396,6 +433,20 @@ void paged_partition_kernel(const DecodeArgs a) {
     __shared__ int s_total[2];  // full partitions, partial ones
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (a.single) {
+        int sq = blockIdx.x / HC;
+        BatchBlocks b = batch_blocks(a.ctx, a.S, a.MB, sq);
+        if (!list_pays<D>(b, a.S, HC)) {
+            for (int it = blockIdx.x; it < a.S * HC; it += gridDim.x) {
+                sq = it / HC;
+                const int sub = it - sq * HC;
+                decode_item<D, NW>(a, sq, sub / a.nhc, sub % a.nhc, 0, 0, b.len);
+                b.len = -1;
+                __syncthreads();  // the item's LDS is free again
+            }
+            return;
+        }
+    }
     const int pb = item_blocks(a.ctx, a.S, a.MB, a.part_blocks, a.share);
     // Blocks of sequence 64 * group + lane, -1 past the batch.
     auto nblk_of = [&](int group) {
@@ -1242,6 +1293,7 @@ constexpr int kWavesV1Wide = 8;
 // Blocks per sequence up to which several rounds of single-pass workgroups
 // run in plain order.
 constexpr int kSingleRoundBlocks = 64;
+constexpr int kListMaxSeqs = 512;
 // Waves per workgroup of a split-K partition.
 #ifndef SWIFTLLM_WAVES_V2
 #define SWIFTLLM_WAVES_V2 4
@@ -1337,13 +1389,14 @@ int decode_v1(void* out, const void* q, const void* kc, const void* vc, const in
         // at the kernel's register count): snake order over the ranked
         // sequences when there are few enough to rank.
         a.snake = sh.S <= kLptMaxSeqs ? cus : 0;
-    } else if (sh.MB > kSingleRoundBlocks && sh.S <= kPartMaxSeqs) {
-        // Several rounds of workgroups, and contexts long enough for the last
-        // ones to leave a tail: the item list, longest first, one item per
-        // sequence and kv head. Measured (us per call, plain order -> list):
-        // lognormal contexts, 32/8 heads x 128, 256 up to 8192 tokens 243 ->
-        // 182, up to 2048 147 -> 131, 140 up to 8192 168 -> 136; 256 of
-        // 1000-4000 413 -> 394; but 256 of 16-128 18.8 -> 28.
+    } else if (sh.MB > kSingleRoundBlocks && sh.S <= kListMaxSeqs) {
+        // Several rounds of workgroups, and tables that may hold contexts long
+        // enough for the last ones to leave a tail: the partition kernel, one
+        // item per sequence and kv head, which takes them longest first where
+        // that pays (list_pays). Of more sequences the list costs more than a
+        // tail of theirs: 600, one of 2500 tokens and the others 32, 48.8 in
+        // plain order, 55.8 by the list.
+        a.single = true;
         a.part_blocks = std::min(sh.MB, 1 << 27);  // 2^31 tokens
         a.share = item_share(a);
         bool too_large = false;

@@ -107,3 +107,14 @@ def test_one_long_context_among_short_ones_is_split(dev, S, long, partition):
     d = _Decode([32] * (S - 1) + [long], 32, 8, 128, (long + 15) // 16)
     split, single = best_us(d.v2(partition)), best_us(d.v1)
     assert split < 0.75 * single, f"{split:.1f} us, single pass {single:.1f} us"
+
+
+@pytest.mark.parametrize("S,H,Hkv,D", [(256, 32, 8, 128), (256, 8, 8, 64), (1024, 8, 8, 64)])
+def test_single_pass_of_short_contexts_under_wide_tables(dev, S, H, Hkv, D):
+    """The table's width is what a program allocates, not what a batch needs:
+    contexts of 16-128 tokens cost about the same under tables for 8192 (they
+    went through a list that each workgroup builds: 27 us against 17, 17.5
+    against 9.3, 65 against 28)."""
+    lens = np.random.default_rng(S).integers(16, 129, size=S)
+    us = [best_us(_Decode(lens, H, Hkv, D, blocks).v1) for blocks in (512, 8)]
+    assert us[0] < 1.4 * us[1], f"{us[0]:.1f} us, tables of 8 blocks {us[1]:.1f} us"
