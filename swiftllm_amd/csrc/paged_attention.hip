@@ -800,19 +800,39 @@ struct StreamArgs {
 // Blocks per sequence -> exclusive prefix in s_pre[0..S] (s_pre[S] = total),
 // clamped context lengths in s_len. All threads of the workgroup take part.
 // A: any argument struct with S, ctx and MB.
+// Returns the longest length; s_most: one entry per wave. Up to 64 sequences are
+// scanned in registers, a lane each, with one barrier.
 template <typename A>
-__device__ __forceinline__ void stream_prefix(const A& a, int* s_pre, int* s_len, int* s_tot) {
+__device__ __forceinline__ int stream_prefix(const A& a, int* s_pre, int* s_len, int* s_tot, int* s_most) {
+    if (a.S <= 64) {
+        const int c = threadIdx.x & 63;
+        const int L0 = c < a.S ? max(a.ctx[c], 0) : 0;
+        const int nb = min((L0 + kBlockTokens - 1) / kBlockTokens, a.MB);
+        const int len = min(L0, nb * kBlockTokens);
+        const int incl = wave_inclusive_scan(nb);
+        if (threadIdx.x < 64 && c < a.S) {
+            s_len[c] = len;
+            s_pre[c] = incl - nb;
+            if (c == a.S - 1) s_pre[a.S] = incl;
+        }
+        __syncthreads();
+        return wave_max(len);
+    }
     const int chunk = (a.S + blockDim.x - 1) / blockDim.x;
     const int c0 = threadIdx.x * chunk;
     int run = 0;
+    int most = 0;
     for (int c = c0; c < min(a.S, c0 + chunk); ++c) {
         const int L0 = max(a.ctx[c], 0);
         const int nb = min((L0 + kBlockTokens - 1) / kBlockTokens, a.MB);
         s_len[c] = min(L0, nb * kBlockTokens);
+        most = max(most, min(L0, nb * kBlockTokens));
         s_pre[c] = run;  // local exclusive prefix, offset added below
         run += nb;
     }
     s_tot[threadIdx.x] = run;
+    most = wave_max(most);
+    if ((threadIdx.x & 63) == 0) s_most[threadIdx.x >> 6] = most;
     __syncthreads();
     if (threadIdx.x < 64) {
         // exclusive scan of the (<= 256) chunk totals by wave 0
@@ -838,7 +858,9 @@ __device__ __forceinline__ void stream_prefix(const A& a, int* s_pre, int* s_len
     __syncthreads();
     const int off = s_tot[threadIdx.x];
     for (int c = c0; c < min(a.S, c0 + chunk); ++c) s_pre[c] += off;
+    for (int w = 0; w < static_cast<int>(blockDim.x) / 64; ++w) most = max(most, s_most[w]);
     __syncthreads();
+    return most;
 }
 
 template <int D>
@@ -849,7 +871,8 @@ void paged_decode_streamk_kernel(const StreamArgs a) {
     int* s_pre = s_dyn;              // [S + 1]
     int* s_len = s_dyn + a.S + 1;    // [S]
     __shared__ int s_tot[64 * kStreamWaves];
-    stream_prefix(a, s_pre, s_len, s_tot);
+    __shared__ int s_most[kStreamWaves];
+    stream_prefix(a, s_pre, s_len, s_tot, s_most);
 
     // Sequences without blocks are not in the list: zero their outputs here.
     for (int sz = blockIdx.x; sz < a.S; sz += gridDim.x) {
@@ -1023,7 +1046,10 @@ __global__ __launch_bounds__(256) void paged_streamk_reduce_kernel(const StreamR
 // most teams + 1 per sequence, whatever partition size the caller asks for.
 // A range that covers a whole sequence writes its output; otherwise its first
 // segment leaves a fragment in the workgroup's even slot and its last one in
-// the odd slot, and paged_team_reduce_kernel combines them.
+// the odd slot, and paged_team_reduce_kernel combines them. Where all contexts
+// are short (team_whole_blocks) the teams take whole sequences instead, one
+// after the other (blocks per team 0: the reduce has nothing to do); the table's
+// width does not tell, so the kernel looks at the lengths.
 //
 // Bound: HBM for long contexts, for short ones the latency of two dependent
 // kernels. Measured on MI355X (us per call, 512-token partitions; before: a
@@ -1040,6 +1066,17 @@ __global__ __launch_bounds__(256) void paged_streamk_reduce_kernel(const StreamR
 constexpr int kTeamWaves = 4;
 constexpr int kTeamPerCU = 2;  // workgroups per CU: two waves per SIMD
 
+// Blocks of the longest context up to which teams take whole sequences. Cut, a
+// context of few sequences spreads over the teams it would leave idle, so the
+// line rises with the sequences per team. Measured with tables 512 blocks wide
+// (us per call, cut / whole, 32/8 heads x 128, 64 teams): 1 sequence of 128
+// tokens 7.7 / 7.2, 192 7.7 / 7.6, 256 7.7 / 8.1; 4 of 256 8.7 / 8.1, 384 8.7 /
+// 9.2; 16 of 384 11.2 / 10.1, 512 11.9 / 11.7; 64 of 16-512 24.7 / 17.5; 96 of
+// 16-128 19.8 / 11.7.
+__device__ __forceinline__ int team_whole_blocks(int S, int teams) {
+    return min((12 + 64 * S / teams) & ~3, 32);
+}
+
 struct TeamArgs {
     f16* out;
     const f16* q;
@@ -1048,7 +1085,7 @@ struct TeamArgs {
     const int* bt;
     const int* ctx;
     float* frag;  // [2 * teams * TS][kFragHead + gstride * D]
-    int* meta;    // for the reduce: [0] blocks per team, [1 .. S + 1] block prefix
+    int* meta;    // for the reduce: [0] blocks per team (0: nothing was cut), [1 .. S + 1] block prefix
     float scale_log2;
     int S, H, Hkv, G, nhc, MB, num_blocks;
     int teams;
@@ -1064,10 +1101,12 @@ void paged_team_kernel(const TeamArgs a) {
     int* s_pre = reinterpret_cast<int*>(smem + merge_lds_floats<D, NW>(a.G));  // [S + 1]
     int* s_len = s_pre + a.S + 1;                                              // [S]
     __shared__ int s_tot[64 * NW];
-    stream_prefix(a, s_pre, s_len, s_tot);
+    __shared__ int s_most[NW];
+    const int most = stream_prefix(a, s_pre, s_len, s_tot, s_most);
 
     const int U = __builtin_amdgcn_readfirstlane(s_pre[a.S]);
-    const int q = (U + a.teams - 1) / a.teams;
+    const bool whole = __builtin_amdgcn_readfirstlane(most) <= team_whole_blocks(a.S, a.teams) * kBlockTokens;
+    const int q = whole ? 0 : (U + a.teams - 1) / a.teams;
     if (blockIdx.x == 0) {
         for (int i = threadIdx.x; i <= a.S; i += blockDim.x) a.meta[1 + i] = s_pre[i];
         if (threadIdx.x == 0) a.meta[0] = q;
@@ -1101,12 +1140,20 @@ void paged_team_kernel(const TeamArgs a) {
         ident[i] = (4 * kg + i == r) ? static_cast<f16>(1.0f) : static_cast<f16>(0.0f);
     }
     const int loff = kv_elem_offset(r, 4 * kg);
-    int u = u0;
-    while (u < u1) {
-        int lo = 0, hi = a.S;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (s_pre[mid] <= u) lo = mid; else hi = mid;
+    int u = u0;           // whole: unused
+    int next = team;      // whole: the team's next sequence
+    bool first = true;    // the workgroup's first segment
+    while (whole ? next < a.S : u < u1) {
+        int lo = next, hi = a.S;
+        if (whole) {
+            next += a.teams;
+            if (s_pre[lo + 1] == s_pre[lo]) continue;
+        } else {
+            lo = 0;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (s_pre[mid] <= u) lo = mid; else hi = mid;
+            }
         }
         // Wave-uniform, in scalar registers, so the block-table reads stay
         // scalar loads.
@@ -1114,8 +1161,8 @@ void paged_team_kernel(const TeamArgs a) {
         const int L = __builtin_amdgcn_readfirstlane(s_len[s]);
         const int pre = __builtin_amdgcn_readfirstlane(s_pre[s]);
         const int nb = __builtin_amdgcn_readfirstlane(s_pre[s + 1]) - pre;
-        const int j0 = u - pre;
-        const int seg = min(nb - j0, u1 - u);
+        const int j0 = whole ? 0 : u - pre;
+        const int seg = whole ? nb : min(nb - j0, u1 - u);
         QOperand<D> qB;
         {
             const f16* qp = a.q + (static_cast<size_t>(s) * a.H + h0 + min(r, gn - 1)) * D + 4 * kg;
@@ -1135,8 +1182,9 @@ void paged_team_kernel(const TeamArgs a) {
                          a.num_blocks, kvh, loff, kg, qB, ident, a.scale_log2);
         const float l_run = sum_over_kg(st.l);
         const bool direct = j0 == 0 && seg == nb;
-        float* f = a.frag + static_cast<size_t>(2 * blockIdx.x + (u != u0)) * (kFragHead + gstride * D);
-        if (u != u0) __syncthreads();  // the segment before has been read from LDS
+        float* f = a.frag + static_cast<size_t>(2 * blockIdx.x + !first) * (kFragHead + gstride * D);
+        if (!first) __syncthreads();  // the segment before has been read from LDS
+        first = false;
         merge_waves<D, NW>(smem, st, l_run, gn, gstride, w, r, kg, [&](int g, int d, float o, float M, float den) {
             if (direct) {
                 a.out[(static_cast<size_t>(s) * a.H + h0 + g) * D + d] = static_cast<f16>(o);
@@ -1169,7 +1217,7 @@ __global__ __launch_bounds__(256) void paged_team_reduce_kernel(const TeamReduce
     const int q = a.meta[0];
     const int pre = a.meta[1 + s];
     const int nb = a.meta[2 + s] - pre;
-    if (nb == 0) return;
+    if (nb == 0 || q == 0) return;
     const int ta = pre / q;
     const int P = (pre + nb - 1) / q - ta + 1;
     if (P == 1) return;  // written by its team

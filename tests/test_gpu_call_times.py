@@ -118,3 +118,15 @@ def test_single_pass_of_short_contexts_under_wide_tables(dev, S, H, Hkv, D):
     lens = np.random.default_rng(S).integers(16, 129, size=S)
     us = [best_us(_Decode(lens, H, Hkv, D, blocks).v1) for blocks in (512, 8)]
     assert us[0] < 1.4 * us[1], f"{us[0]:.1f} us, tables of 8 blocks {us[1]:.1f} us"
+
+
+@pytest.mark.parametrize("S", [64, 96])
+@pytest.mark.parametrize("partition", [512, 0])
+def test_split_of_short_contexts_under_wide_tables(dev, S, partition):
+    """Teams do not cut contexts of 16-128 tokens: a split call takes them whole
+    and costs one empty kernel more than the single pass (96 of them 19.5 us
+    cut, 11.7 whole, single pass 10.9)."""
+    lens = np.random.default_rng(S).integers(16, 129, size=S)
+    d = _Decode(lens, 32, 8, 128, 512)
+    split, single = best_us(d.v2(partition)), best_us(d.v1)
+    assert split < 1.5 * single, f"{split:.1f} us, single pass {single:.1f} us"
