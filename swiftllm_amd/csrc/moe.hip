@@ -153,7 +153,7 @@ __device__ __forceinline__ void select_topk(const float* row, int E, float (&bv)
 // holds logits j, j + 16, ... (N of them at most) as integers in the logits'
 // order, and K passes each take the row's maximum and then the lowest index
 // that has it, two chains of four DPP steps. Every lane of the row ends with
-// the K picks. Requires logits without NaN; `row` is null for rows past T.
+// the K picks. Requires logits without NaN.
 __device__ __forceinline__ int ordered(float x) {
     const int b = __builtin_bit_cast(int, x + 0.0f);  // -0 ranks as 0
     return b ^ ((b >> 31) & 0x7fffffff);
@@ -192,9 +192,10 @@ __device__ __forceinline__ void select_topk_row(const float (&v)[N], int E, int 
     }
 }
 
-// Routes token t (16 lanes per token, j the lane's place) for E > 16: ids in
-// bi, and ids and weights written by the row's first lanes. A wave that holds
-// a NaN routes with the one-thread selection, whose order then counts.
+// Routes token t (16 lanes per token, j the lane's place; a token past T as the
+// last one) for E > 16: ids in bi, and ids and weights written by the row's
+// first lane if t < T. A wave that holds a NaN routes with the one-thread
+// selection, whose order then counts.
 template <int K, int N>
 __device__ __forceinline__ void route_row(const RouteArgs& a, int t, int j, int (&bi)[K]) {
     const bool live = t < a.T;

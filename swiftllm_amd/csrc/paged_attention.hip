@@ -115,8 +115,8 @@ __device__ __forceinline__ void attend_blocks(WaveState<D>& st, const const_int*
     }
 }
 
-// The sequence with the r-th longest context (ties by index), found by every
-// workgroup of a single-pass grid that is resident all at once (the snake
+// The sequence with the r-th longest context (ties by index) of at most
+// kLptMaxSeqs, found by every workgroup of a single-pass grid that is resident all at once (the snake
 // order below). Each thread ranks S / 256 sequences against all S, so the
 // cost grows as S^2: measured on MI355X with the ranking in every grid,
 // 1024 sequences of 32-128 tokens took 1324 us against 67 us in plain order,
@@ -127,8 +127,7 @@ __device__ __forceinline__ void attend_blocks(WaveState<D>& st, const const_int*
 constexpr int kLptMaxSeqs = 128;
 
 __device__ __forceinline__ int sequence_for_block(const int* ctx, int S, int r) {
-    if (S > kLptMaxSeqs) return r;
-    __shared__ int s_ctx[kLptMaxSeqs > 0 ? kLptMaxSeqs : 1];
+    __shared__ int s_ctx[kLptMaxSeqs];
     __shared__ int s_seq;
     for (int c = threadIdx.x; c < S; c += blockDim.x) s_ctx[c] = ctx[c];
     if (threadIdx.x == 0) s_seq = r;
@@ -331,10 +330,10 @@ void paged_decode_kernel(const DecodeArgs a) {
 // the list is the order the items start in: first every full partition (of
 // item_blocks() blocks), then the last, partial partition of each sequence in
 // kLptClasses length classes, longest first (an empty sequence's item, which
-// writes zeros, is a partial of length 0). A single-pass call with many
-// sequences takes the same list with one partition per sequence. Measured with the gather kernel
-// of libswiftllm_ceilings on config 4's items at 1024-token partitions:
-// 151 us longest first against 166 us in sequence order.
+// writes zeros, is a partial of length 0). A single-pass call of several rounds
+// may take the same list with one partition per sequence (list_pays). Measured
+// with the gather kernel of libswiftllm_ceilings on config 4's items at
+// 1024-token partitions: 151 us longest first against 166 us in sequence order.
 //
 // The item of one list position is run by several workgroups (one per kv-head
 // chunk), each with its own copy of the list, so the list must come out the
@@ -547,11 +546,13 @@ void paged_partition_kernel(const DecodeArgs a) {
 // aligned); out(d, v) stores one output.
 // One wave combines a head: no barriers, lane l owns outputs
 // [l * D / 64, (l + 1) * D / 64), so every fragment row is one coalesced load.
-// The rows of the first CH fragments are loaded before the headers (max and
-// sum) of the first 64, all in flight together, so the combine pays one
-// memory latency per CH fragments; rows past the last fragment re-read it
-// and get weight 0. The weights live one per lane and are broadcast with
-// readlane; the rows are added in fragment order.
+// The rows of the first kReduceRows fragments are loaded before the headers
+// (max and sum) of the first 64, all in flight together, so the combine pays
+// one memory latency per kReduceRows fragments; rows past the last fragment
+// re-read it and get weight 0. The weights live one per lane and are broadcast
+// with readlane; the rows are added in fragment order.
+constexpr int kReduceRows = 16;
+
 template <int D>
 __device__ __forceinline__ void load_row(const float* p, float (&v)[D / 64]) {
     if constexpr (D == 128) {
@@ -567,9 +568,9 @@ __device__ __forceinline__ float readlane_f(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 
-template <int D, int CH, typename FM, typename FL, typename FO, typename OUT>
+template <int D, typename FM, typename FL, typename FO, typename OUT>
 __device__ __forceinline__ void combine_head_wave(int P, FM fm, FL fl, FO fo, OUT out) {
-    static_assert(CH == 16 || CH == 64, "rows per load batch");
+    constexpr int CH = kReduceRows;
     constexpr int DL = D / 64;
     const int lane = threadIdx.x & 63;
     if (P <= 0) {
@@ -619,20 +620,16 @@ __device__ __forceinline__ void combine_head_wave(int P, FM fm, FL fl, FO fo, OU
     for (int j = 0; j < DL; ++j) out(lane * DL + j, acc[j] * inv);
 }
 
-// Fragment rows per load batch of a head's combine: 16 for up to 16
-// fragments, else 64 (128 registers of rows at D = 128).
-constexpr int kReduceSmall = 16;
-
 // The same combine by the NW waves of a workgroup, for heads with many
 // fragments: wave w takes the 16-fragment chunks w, w + NW, ..., keeping a
 // running max, sum and rescaled partial over its chunks (one memory latency
 // per chunk, its 16 rows loaded before the headers), and wave 0 merges the
 // NW partials through LDS. A head then costs ceil(P / (16 NW)) latencies
-// instead of ceil(P / 64), with NW times the waves in flight.
+// instead of ceil(P / 16), with NW times the waves in flight.
 template <int D, int NW, typename FM, typename FL, typename FO, typename OUT>
 __device__ __forceinline__ void combine_head_split(int P, FM fm, FL fl, FO fo, OUT out) {
     constexpr int DL = D / 64;
-    constexpr int CH = 16;
+    constexpr int CH = kReduceRows;
     __shared__ float s_acc[NW][D];
     __shared__ float s_md[NW][2];
     const int lane = threadIdx.x & 63;
@@ -717,9 +714,9 @@ struct ReduceArgs {
     float share;
 };
 
-// Combine of head h of sequence s; CH: fragment rows per load batch of the
-// one-wave combine, 0: the four waves of the workgroup (combine_head_split).
-template <int D, int CH>
+// Combine of head h of sequence s by one wave, or by the four waves of the
+// workgroup (SPLIT).
+template <int D, bool SPLIT>
 __device__ __forceinline__ void reduce_head(const ReduceArgs& a, int s, int h) {
     const int L = max(a.ctx[s], 0);
     const int nblk = min((L + kBlockTokens - 1) / kBlockTokens, a.MB);
@@ -736,27 +733,26 @@ __device__ __forceinline__ void reduce_head(const ReduceArgs& a, int s, int h) {
     auto fl = [&](int p) { return pl[p]; };
     auto fo = [&](int p) { return po + static_cast<size_t>(p) * D; };
     auto out = [&](int d, float v) { o[d] = static_cast<f16>(v); };
-    if constexpr (CH == 0) {
+    if constexpr (SPLIT) {
         combine_head_split<D, 4>(nparts, fm, fl, fo, out);
     } else {
-        combine_head_wave<D, CH>(nparts, fm, fl, fo, out);
+        combine_head_wave<D>(nparts, fm, fl, fo, out);
     }
 }
 
-// One wave per (query head, sequence), four heads per workgroup; CH fragment
-// rows per load batch.
-template <int D, int CH>
+// One wave per (query head, sequence), four heads per workgroup.
+template <int D>
 __global__ __launch_bounds__(256) void paged_reduce_wave_kernel(const ReduceArgs a) {
     const int h = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (h >= a.H) return;
-    reduce_head<D, CH>(a, blockIdx.y, h);
+    reduce_head<D, false>(a, blockIdx.y, h);
 }
 
 // One (query head, sequence) per workgroup of four waves, for more than 16
 // partitions per sequence.
 template <int D>
 __global__ __launch_bounds__(256) void paged_reduce_split_kernel(const ReduceArgs a) {
-    reduce_head<D, 0>(a, blockIdx.y, blockIdx.x);
+    reduce_head<D, true>(a, blockIdx.y, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1029,7 +1025,7 @@ __global__ __launch_bounds__(256) void paged_streamk_reduce_kernel(const StreamR
         return a.frag + slot * fs;
     };
     f16* o = a.out + (static_cast<size_t>(s) * a.H + kvh * a.G + g0 + g) * D;
-    combine_head_wave<D, kReduceSmall>(
+    combine_head_wave<D>(
         P, [&](int i) { return frag_of(i)[g]; }, [&](int i) { return frag_of(i)[16 + g]; },
         [&](int i) { return frag_of(i) + kFragHead + static_cast<size_t>(g) * D; },
         [&](int d, float v) { o[d] = static_cast<f16>(v); });
@@ -1349,16 +1345,15 @@ constexpr int kListMaxSeqs = 512;
 constexpr int kWavesV2 = SWIFTLLM_WAVES_V2;
 
 template <int D, int NW>
-hipError_t launch_decode_t(const DecodeArgs& a, int S, int mp_grid, hipStream_t stream) {
+hipError_t launch_decode_t(const DecodeArgs& a, hipStream_t stream) {
     const size_t lds = static_cast<size_t>(merge_lds_floats<D, NW>(a.G)) * sizeof(float);
-    dim3 grid(mp_grid, a.Hkv * a.nhc, S);
+    const dim3 grid(1, a.Hkv * a.nhc, a.S);
     return launch(paged_decode_kernel<D, NW>, grid, dim3(NW * 64), lds, stream, a);
 }
 
 template <int NW>
-hipError_t launch_decode(const DecodeArgs& a, int D, int S, int mp_grid, hipStream_t stream) {
-    return D == 128 ? launch_decode_t<128, NW>(a, S, mp_grid, stream)
-                    : launch_decode_t<64, NW>(a, S, mp_grid, stream);
+hipError_t launch_decode(const DecodeArgs& a, int D, hipStream_t stream) {
+    return D == 128 ? launch_decode_t<128, NW>(a, stream) : launch_decode_t<64, NW>(a, stream);
 }
 
 template <int D, int NW>
@@ -1430,7 +1425,7 @@ int decode_v1(void* out, const void* q, const void* kc, const void* vc, const in
     // 12.5 -> 11.4, 32 x 512 13.9 -> 12.4, 4 x 2048 of 8 heads x 64 16.5 ->
     // 13.7. At 64 x 32-512 (512 items) 15.8 -> 18.5, so not beyond.
     if (items <= cus && a.G <= 8) {
-        return launched(launch_decode<kWavesV1Wide>(a, sh.D, sh.S, 1, stream), who);
+        return launched(launch_decode<kWavesV1Wide>(a, sh.D, stream), who);
     }
     if (items <= 3LL * cus) {
         // The whole grid is resident at once (three 4-wave workgroups per CU
@@ -1450,7 +1445,7 @@ int decode_v1(void* out, const void* q, const void* kc, const void* vc, const in
         bool too_large = false;
         return launched(launch_partition<kWavesV2>(a, sh.D, stream, &too_large), who);
     }
-    return launched(launch_decode<kWavesV1>(a, sh.D, sh.S, 1, stream), who);
+    return launched(launch_decode<kWavesV1>(a, sh.D, stream), who);
 }
 
 // Whether a split-K call runs single pass instead: its tables are too short
@@ -1538,12 +1533,12 @@ TeamNeed team_need(const Shape& sh, int cus) {
     return n;
 }
 
-// A wave combines a head in one batch of kReduceSmall rows for up to that
-// many partitions per sequence; beyond, the four waves of a workgroup do.
+// A wave combines a head in one batch of kReduceRows rows for up to that many
+// partitions per sequence; beyond, the four waves of a workgroup do.
 template <int D>
 hipError_t launch_reduce_t(const ReduceArgs& r, int S, hipStream_t stream) {
-    if (r.MP <= kReduceSmall) {
-        return launch(paged_reduce_wave_kernel<D, kReduceSmall>, dim3((r.H + 3) / 4, S), dim3(256), 0, stream, r);
+    if (r.MP <= kReduceRows) {
+        return launch(paged_reduce_wave_kernel<D>, dim3((r.H + 3) / 4, S), dim3(256), 0, stream, r);
     }
     return launch(paged_reduce_split_kernel<D>, dim3(r.H, S), dim3(256), 0, stream, r);
 }
