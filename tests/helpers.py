@@ -6,7 +6,8 @@ from __future__ import annotations
 import numpy as np
 
 from swiftllm_amd import paged_attention as pa
-from swiftllm_amd._hip import DeviceArray, synchronize
+from swiftllm_amd import workloads
+from swiftllm_amd._hip import DeviceArray, cu_count, synchronize
 
 # Attention tolerance against the fp64 oracle (fp16 in/out, fp32 accumulate):
 # max |out - ref| <= 2e-3 and max |out - ref| / max(|ref|, 1e-3) <= 1e-2.
@@ -46,6 +47,53 @@ def assert_gemm_close(gpu, ref, what=""):
     bound = 2.0 ** -10 * np.abs(ref) + 1e-3 * rms
     worst = float((err - bound).max()) if err.size else -1.0
     assert worst <= 0, f"{what}: max err {err.max():.3e}, rms {rms:.3e}"
+
+
+def split_route(w, ps):
+    """The kernel a split-K call on this workload runs, by the launcher's rules
+    (single_pass, team_need and effective_partition of paged_attention.hip):
+    "single", "teams", "items" or "balanced". Tests state the one they are for,
+    so that a rule that moves does not leave them on another."""
+    sh, cus = w.shape, cu_count()
+    S, H, Hkv, D, MB = (sh[k] for k in ("num_seqs", "num_heads", "num_kv_heads", "head_dim",
+                                        "max_num_blocks_per_seq"))
+    G = H // Hkv
+    TS = Hkv * ((G + 15) // 16)
+    if ps == 0 and (S > 4096 or 4 * TS > 12 * cus):
+        ps = 512
+    items = S * TS
+    if S <= 4096:
+        line = (32 if ps == 0 and items > 4 * cus else 64) if items > 3 * cus else \
+            min(32 + items // 4, 64 if ps == 0 else 96)
+        if MB <= line:
+            return "single"
+    teams = 2 * cus // TS
+    need = (8 * teams * TS * (32 + min(16, G) * D) + 255) // 256 * 256 + 4 * (S + 2)
+    if teams >= 4 and S <= min(2 * teams, 4096) and \
+            (ps == 0 or need <= pa.paged_attention_v2_workspace_size(S, H, Hkv, D, 16, MB, ps)):
+        return "teams"
+    return "balanced" if ps == 0 else "items"
+
+
+def item_fragments(w, ps):
+    """Fragments per head of each sequence in the item kernel: items of
+    item_blocks() blocks, whole partitions up to one and a half shares of a
+    resident workgroup."""
+    sh = w.shape
+    G = sh["num_heads"] // sh["num_kv_heads"]
+    blocks = np.minimum((np.maximum(w.context_lens, 0) + 15) // 16, sh["max_num_blocks_per_seq"])
+    share = np.float32(1.5) * np.float32(sh["num_kv_heads"] * ((G + 15) // 16)) / np.float32(3 * cu_count())
+    pb = ps // 16 * max(1, int(np.float32(blocks.sum()) * share) // (ps // 16))
+    return -(-blocks // pb)
+
+
+def padded(w, mb):
+    """The same batch with block tables mb wide (the width is what the launcher
+    sees of the lengths)."""
+    bt = np.zeros((w.block_tables.shape[0], mb), np.int32)
+    bt[:, :w.block_tables.shape[1]] = w.block_tables
+    return workloads.DecodeWorkload("padded", w.q, w.key_cache, w.value_cache, bt, w.context_lens,
+                                    w.scale)
 
 
 def expert_offsets(rng, E, m_total, empty=()):

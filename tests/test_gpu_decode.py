@@ -9,10 +9,11 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import DeviceWorkload, assert_attention_close
+from helpers import (DeviceWorkload, assert_attention_close, item_fragments, padded,
+                     split_route)
 from swiftllm_amd import paged_attention as pa
 from swiftllm_amd import workloads
-from swiftllm_amd._hip import DeviceArray, synchronize
+from swiftllm_amd._hip import DeviceArray, cu_count, synchronize
 
 pytestmark = pytest.mark.gpu
 
@@ -28,7 +29,7 @@ def test_config1_tiny_mha(dev, variant, ps):
     assert_attention_close(out, _ref(w), f"config1 {variant} ps={ps}")
 
 
-# 512: one wave per partition; 1024: two; 2048: the whole 4-wave workgroup
+# 64 sequences: teams at every partition size
 @pytest.mark.parametrize("variant,ps", [("v1", None), ("v2", 512), ("v2", 1024), ("v2", 2048),
                                         ("v2", 0)])
 def test_config2_llama3_8b(dev, variant, ps):
@@ -95,6 +96,12 @@ def test_gqa_groups(dev, H, Hkv, D):
     ref = _ref(w)
     for variant, ps in (("v1", None), ("v2", 32), ("v2", 0)):
         assert_attention_close(dw.run(variant, partition_size=ps), ref, f"H{H} Hkv{Hkv} D{D} {variant} ps={ps}")
+    # tables past every single-pass line: the team kernel, which cuts the longest
+    w = padded(w, 300)
+    dw = DeviceWorkload(w)
+    for ps in (32, 0):
+        assert split_route(w, ps) == "teams"
+        assert_attention_close(dw.run("v2", partition_size=ps), ref, f"teams H{H} Hkv{Hkv} D{D} ps={ps}")
 
 
 def _poisoned(rng, S, ctx, D=128, H=32, Hkv=8, MB=None):
@@ -119,12 +126,16 @@ def _poisoned(rng, S, ctx, D=128, H=32, Hkv=8, MB=None):
     return workloads.DecodeWorkload("poison", q, kc, vc, bt, ctx.astype(np.int32), 1.0 / np.sqrt(D))
 
 
-@pytest.mark.parametrize("variant,ps", [("v1", None), ("v2", 16), ("v2", 48), ("v2", 0)])
-def test_edge_context_lengths(dev, variant, ps):
-    """ctx in {0, 1, 15, 16, 17, 31, 33, 200}; unused slots hold NaN."""
+@pytest.mark.parametrize("variant,ps,long,route", [
+    ("v1", None, 200, None), ("v2", 16, 200, "single"), ("v2", 48, 200, "single"), ("v2", 0, 200, "single"),
+    ("v2", 48, 1700, "teams"), ("v2", 0, 1700, "teams"), ("v2", 16, 2100, "teams"),
+])
+def test_edge_context_lengths(dev, variant, ps, long, route):
+    """ctx in {0, 1, 15, 16, 17, 31, 33, 200 or more}; unused slots hold NaN."""
     rng = np.random.default_rng(7)
-    ctx = np.array([0, 1, 15, 16, 17, 31, 33, 200], np.int32)
+    ctx = np.array([0, 1, 15, 16, 17, 31, 33, long], np.int32)
     w = _poisoned(rng, len(ctx), ctx)
+    assert route is None or split_route(w, ps) == route
     out = DeviceWorkload(w).run(variant, partition_size=ps)
     ref = _ref(w)
     assert np.all(out[0] == 0), "context 0 must give zeros"
@@ -339,15 +350,14 @@ def _random_batch(rng, lens, H, Hkv, D, std=1.0, extra_blocks=4):
 
 @pytest.mark.parametrize("G", [8, 1])
 def test_one_long_sequence_many_fragments(dev, G):
-    """One 32768-token sequence (plus a short one) in balanced mode: the
-    sequence spans hundreds of teams, so its reduce combines more than 64
-    fragments per item (several passes of the one-wave combine); the
-    partitioned modes combine 64 and 8 partitions (workgroup reduce)."""
+    """One 32768-token sequence (plus a short one): the teams cut it into 64
+    ranges, 4096-token partitions have no room for them and leave 8 items."""
     rng = np.random.default_rng(70 + G)
     w = _random_batch(rng, [32768, 37], H=8 * G, Hkv=8, D=128)
     dw = DeviceWorkload(w)
     ref = _ref(w)
-    for ps in (0, 512, 4096):
+    for ps, route in ((0, "teams"), (512, "teams"), (4096, "items")):
+        assert split_route(w, ps) == route
         assert_attention_close(dw.run("v2", partition_size=ps), ref, f"long G={G} ps={ps}")
 
 
@@ -369,10 +379,10 @@ def context_128k(dev):
 
 @pytest.mark.parametrize("variant,ps", [("v1", None), ("v2", 512), ("v2", 16), ("v2", 0)])
 def test_context_past_128k(context_128k, variant, ps):
-    """The single pass over 8,193 blocks; split-K with 257 partitions of 512
-    tokens and with 8,193 of 16 (the workgroup reduce's chunked loop many
-    times over, and an 818 MB workspace); balanced mode."""
+    """The single pass over 8,193 blocks; the teams' ranges of them, at 512- and
+    16-token partitions (an 818 MB workspace) and in balanced mode."""
     dw, ref = context_128k
+    assert variant == "v1" or split_route(dw.w, ps) == "teams"
     assert_attention_close(dw.run(variant, partition_size=ps), ref, f"128k {variant} ps={ps}")
 
 
@@ -393,20 +403,23 @@ def test_more_sequences_than_the_lds_tables(dev):
         assert_attention_close(out[live], ref[live], f"4500 seqs {variant} ps={ps}")
 
 
-@pytest.mark.parametrize("S,ps", [(300, 64), (1100, 32), (4096, 16)])
-def test_partition_items_longest_first_cover_every_partition(dev, S, ps):
+@pytest.mark.parametrize("S,H,Hkv,median,ps", [(300, 32, 8, 90.0, 64), (1100, 8, 2, 90.0, 32),
+                                               (4096, 8, 2, 12.0, 16)])
+def test_partition_items_longest_first_cover_every_partition(dev, S, H, Hkv, median, ps):
     """The split-K kernel orders its items longest first in a list that every
     workgroup builds in its own LDS; the items of one list position are run
     by different workgroups (one per kv head), so the list must come out the
-    same in each. Ragged batches of more than one 256-sequence chunk, at
-    partitions small enough that every workgroup walks many items and every
-    length class holds ties, with empty sequences: every partition of every
-    sequence is attended exactly once (a missing one leaves the output
-    unwritten or the reduce short of a fragment)."""
+    same in each. Ragged batches of several groups of 64 sequences, at
+    partitions small enough that the longest sequences have full items and a
+    partial one and that every length class holds ties, with empty sequences:
+    every partition of every sequence is attended exactly once (a missing one
+    leaves the output unwritten or the reduce short of a fragment)."""
     rng = np.random.default_rng(S + ps)
-    lens = np.clip(np.rint(np.exp(rng.normal(np.log(90.0), 1.0, size=S))), 0, 1500).astype(np.int64)
+    lens = np.clip(np.rint(np.exp(rng.normal(np.log(median), 1.0, size=S))), 0, 1500).astype(np.int64)
     lens[rng.choice(S, size=S // 10, replace=False)] = 0
-    w = _random_batch(rng, lens, H=8, Hkv=2, D=64)
+    lens[:2] = [1500, 1477]
+    w = _random_batch(rng, lens, H=H, Hkv=Hkv, D=64)
+    assert split_route(w, ps) == "items" and item_fragments(w, ps).max() >= 2
     out = DeviceWorkload(w).run("v2", partition_size=ps)
     live = lens > 0
     assert np.all(out[~live] == 0), "empty sequences must be zero"
@@ -414,16 +427,13 @@ def test_partition_items_longest_first_cover_every_partition(dev, S, ps):
 
 
 @pytest.mark.parametrize("H,Hkv,D", [(64, 8, 128), (64, 2, 128), (48, 2, 128), (16, 1, 128), (32, 8, 64)])
-def test_partition_streams_ragged(dev, H, Hkv, D):
-    """Split-K over short partitions of a batch with few sequences runs as
-    partition streams: equal block ranges per team of waves, cut at partition
-    ends and at range boundaries. Ragged contexts with empty sequences put
-    range boundaries inside partitions, at partition starts and at sequence
-    starts; 16-token partitions make every block a partition, and the 2-kv-head
-    layouts (G = 32, two head chunks; G = 24, the second chunk 8 heads wide)
-    give small teams whose ranges are shorter than a partition; G = 16 with
-    one kv head gives one-wave teams. Pieces that end inside a wave's range
-    are held in LDS and written with the wave's last piece."""
+def test_teams_ragged(dev, H, Hkv, D):
+    """Split-K of a batch with few sequences runs by teams, whatever the
+    partition size: equal block ranges per team of workgroups. Ragged contexts
+    with empty sequences put range boundaries inside sequences and at their
+    starts; the 2-kv-head layouts (G = 32, two head chunks; G = 24, the second
+    chunk 8 heads wide) give small teams with short ranges, G = 16 with one kv
+    head teams of one workgroup."""
     rng = np.random.default_rng(H + Hkv + D)
     S = 40
     lens = np.clip(np.rint(np.exp(rng.normal(np.log(1500.0), 1.2, size=S))), 1, 20000).astype(np.int64)
@@ -433,72 +443,57 @@ def test_partition_streams_ragged(dev, H, Hkv, D):
     ref = _ref(w)
     live = lens > 0
     for ps in (16, 256, 512, 1024):
+        assert split_route(w, ps) == "teams"
         out = dw.run("v2", partition_size=ps)
         assert np.all(out[~live] == 0), f"ps={ps}: empty sequences must be zero"
-        assert_attention_close(out[live], ref[live], f"streams H{H} Hkv{Hkv} D{D} ps={ps}")
+        assert_attention_close(out[live], ref[live], f"teams H{H} Hkv{Hkv} D{D} ps={ps}")
 
 
 @pytest.mark.parametrize("D", [128, 64])
-def test_item_reduce_many_partitions(dev, D):
-    """Split-K over the item kernel (80 sequences: more than a quarter of the
-    teams a partition stream needs) with up to 188 partitions per sequence:
-    above 16 partitions the reduce runs on four waves per head (16, 64), at
-    most 16 on one wave (256); empty and one-block sequences included."""
-    rng = np.random.default_rng(91 + D)
-    S = 80
-    lens = np.clip(np.rint(np.exp(rng.normal(np.log(700.0), 1.0, size=S))), 1, 3000).astype(np.int64)
-    lens[:3] = [0, 1, 3000]
-    w = _random_batch(rng, lens, H=32, Hkv=8, D=D)
-    dw = DeviceWorkload(w)
-    ref = _ref(w)
+@pytest.mark.parametrize("blocks,fragments", [(34, 17), (128, 64), (130, 65), (2000, 223)])
+def test_item_reduce_many_partitions(dev, D, blocks, fragments):
+    """Split-K over the item kernel with one long context among 519 of a block
+    or none: its heads' reduce runs on four waves, over just more than a wave's
+    16-fragment chunk, at and past one pass of the four and several passes."""
+    rng = np.random.default_rng(91 + D + blocks)
+    lens = rng.integers(1, 17, size=520)
+    lens[:3] = [0, 16 * blocks - 5, 0]
+    w = padded(_random_batch(rng, lens, H=4, Hkv=2, D=D), 3000)
+    assert split_route(w, 16) == "items" and item_fragments(w, 16).max() == fragments
+    out = DeviceWorkload(w).run("v2", partition_size=16)
     live = lens > 0
-    for ps in (16, 64, 256):
-        out = dw.run("v2", partition_size=ps)
-        assert np.all(out[~live] == 0), f"ps={ps}: empty sequences must be zero"
-        assert_attention_close(out[live], ref[live], f"item reduce D{D} ps={ps}")
+    assert np.all(out[~live] == 0), "empty sequences must be zero"
+    assert_attention_close(out[live], _ref(w)[live], f"item reduce D{D} {fragments} fragments")
 
 
 @pytest.mark.parametrize("D", [128, 64])
-def test_partition_stream_reduce_fragment_counts(dev, D):
-    """The reduce of a head with more than 16 fragments runs on four waves,
-    each combining 16-fragment chunks, merged through LDS. With 16-token
-    partitions every block is a partition and every range boundary falls on a
-    partition start, so a sequence of n blocks leaves exactly n fragments per
-    head. The counts cross a wave's chunk (16 / 17), one pass of the four
-    waves (63 / 64 / 65) and several passes (129, 200), beside sequences of 1
-    block (written directly), 2 and 8 blocks and an empty one; some last
-    blocks are partial."""
+def test_team_ranges_of_uneven_sequences(dev, D):
+    """Teams of 9 blocks over sequences of 1 to 200 blocks: some inside one
+    range (written directly), some cut into up to 24 fragments, one empty,
+    some last blocks partial."""
     rng = np.random.default_rng(77 + D)
     blocks = np.array([1, 2, 8, 9, 16, 17, 63, 64, 65, 129, 200, 0])
     lens = blocks * 16 - (np.arange(len(blocks)) % 3) * 5
     lens[blocks == 0] = 0
     w = _random_batch(rng, lens, H=64, Hkv=8, D=D)
+    assert split_route(w, 16) == "teams"
     out = DeviceWorkload(w).run("v2", partition_size=16)
     live = lens > 0
     assert np.all(out[~live] == 0), "empty sequences must be zero"
-    assert_attention_close(out[live], _ref(w)[live], f"reduce fragment counts D{D}")
-
-
-def _padded(w, mb):
-    """The same batch with block tables mb wide (the width is what the
-    launcher sees of the lengths)."""
-    bt = np.zeros((w.block_tables.shape[0], mb), np.int32)
-    bt[:, :w.block_tables.shape[1]] = w.block_tables
-    return workloads.DecodeWorkload("padded", w.q, w.key_cache, w.value_cache, bt, w.context_lens,
-                                    w.scale)
+    assert_attention_close(out[live], _ref(w)[live], f"team ranges D{D}")
 
 
 @pytest.mark.parametrize("H,Hkv,D,S", [
     (32, 8, 128, 1), (32, 8, 128, 7), (64, 8, 128, 40), (8, 8, 64, 128),  # teams: up to 2 sequences each
     (8, 8, 64, 129),                       # one more: items
     (48, 2, 128, 5), (16, 1, 64, 300),     # two head chunks, the second 8 wide; one-member teams
-    (128, 128, 64, 8), (256, 256, 64, 3),  # 4 teams; too few: items / streams
+    (128, 128, 64, 8), (256, 256, 64, 3),  # 4 teams; too few: items / balanced
 ])
 def test_split_routes_agree_with_single_pass(dev, H, Hkv, D, S):
-    """Tables padded past every single-pass limit send split-K calls to the
-    teams (few sequences) or the item list (many), narrow ones to the single
-    pass; all against the oracle, with empty, one-token and block-edge
-    contexts, NaN in unused slots and an out-of-pool block."""
+    """Tables padded past every single-pass line send split-K calls to the
+    teams (few sequences) or to the item list and the balanced ranges (many),
+    narrow ones to the single pass; all against the oracle, with empty,
+    one-token and block-edge contexts and NaN in unused slots."""
     rng = np.random.default_rng(H + 7 * Hkv + D + S)
     lens = np.clip(np.rint(np.exp(rng.normal(np.log(120.0), 1.2, size=S))), 0, 900).astype(np.int64)
     edge = np.array([0, 1, 15, 16, 17, 900])[:max(S - 1, 0)]
@@ -514,7 +509,10 @@ def test_split_routes_agree_with_single_pass(dev, H, Hkv, D, S):
     ref = _ref(w)
     live = lens > 0
     for mb in (w.block_tables.shape[1], 3000):
-        dw = DeviceWorkload(_padded(w, mb))
+        wide = padded(w, mb)
+        few = S <= 2 * (2 * cu_count() // (Hkv * ((H // Hkv + 15) // 16))) and Hkv < 256
+        assert mb < 3000 or split_route(wide, 0) == ("teams" if few else "balanced")
+        dw = DeviceWorkload(wide)
         for variant, ps in (("v1", None), ("v2", 16), ("v2", 512), ("v2", 0)):
             out = dw.run(variant, partition_size=ps)
             assert np.all(out[~live] == 0), f"MB={mb} {variant} {ps}: empty sequences must be zero"
@@ -523,15 +521,17 @@ def test_split_routes_agree_with_single_pass(dev, H, Hkv, D, S):
 
 @pytest.mark.parametrize("ps", [16, 64, 512])
 def test_items_of_several_partitions(dev, ps):
-    """More sequences than teams, long tables: an item takes several
-    partitions of the batch, and the reduce has to cut the sequences the same
-    way; up to 188 partitions per sequence (the four-wave reduce) and 6 (one
-    wave)."""
+    """More sequences than two per team, long tables: an item takes several
+    partitions of the batch (96 to 126 blocks here), and the reduce has to cut
+    the sequences the same way: the longest in two, which the four waves
+    reduce where the workspace has more than 16 partitions a sequence (16- and
+    64-token ones), one wave at 512."""
     rng = np.random.default_rng(19 + ps)
     S = 140
     lens = np.clip(np.rint(np.exp(rng.normal(np.log(500.0), 1.2, size=S))), 1, 3000).astype(np.int64)
     lens[:4] = [0, 1, 3000, 2999]
     w = _random_batch(rng, lens, H=32, Hkv=8, D=64)
+    assert split_route(w, ps) == "items" and item_fragments(w, ps).max() == 2
     out = DeviceWorkload(w).run("v2", partition_size=ps)
     live = lens > 0
     assert np.all(out[~live] == 0)
@@ -544,7 +544,74 @@ def test_team_fragment_counts(dev, counts):
     (ranges that end on, before and after a sequence's end)."""
     rng = np.random.default_rng(sum(counts))
     lens = np.array([16 * c - (i % 3) * 5 for i, c in enumerate(counts)])
-    w = _padded(_random_batch(rng, lens, H=64, Hkv=8, D=128), 3000)
+    w = padded(_random_batch(rng, lens, H=64, Hkv=8, D=128), 3000)
     dw = DeviceWorkload(w)
     for ps in (512, 0):
+        assert split_route(w, ps) == "teams"
         assert_attention_close(dw.run("v2", partition_size=ps), _ref(w), f"teams {counts} ps={ps}")
+
+
+@pytest.mark.parametrize("lens,ps,route", [
+    ([160, 40, 33, 16, 300, 0], 512, "teams"),           # whole sequences
+    ([160, 2000, 33, 16, 1500, 0], 512, "teams"),        # cut
+    ([160, 40, 33, 16, 1500, 0] * 25, 64, "items"),
+    ([160, 40, 33, 16, 1500, 0] * 25, 0, "balanced"),
+])
+@pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (136, 8, 64)])  # the second: two head chunks, 16 and 1
+def test_out_of_pool_blocks_skipped_by_every_split_kernel(dev, H, Hkv, D, lens, ps, route):
+    """A block id outside the pool at a sequence's start, inside it or at its
+    end contributes nothing: the rest of the sequence is attended as if the
+    block were not there, and a sequence of such blocks alone gives zeros."""
+    rng = np.random.default_rng(H + len(lens))
+    lens = np.array(lens)
+    w = padded(_random_batch(rng, lens, H, Hkv, D), 300)
+    assert split_route(w, ps) == route
+    NB = w.key_cache.shape[0]
+    kept = w.block_tables.copy()
+    left = lens.copy()
+    for s in range(len(lens)):
+        n = (lens[s] + 15) // 16
+        bad = {0: [0], 1: [n // 2], 2: [n - 1], 3: range(n), 4: [0, 1, n - 2]}.get(s % 6, [])
+        good = [j for j in range(n) if j not in bad]
+        kept[s, :len(good)] = w.block_tables[s, good]
+        left[s] = 16 * len(good) - (16 * n - lens[s] if n - 1 in good else 0)
+        w.block_tables[s, list(bad)] = NB + rng.integers(0, 1000, len(bad))
+    out = DeviceWorkload(w).run("v2", partition_size=ps)
+    ref = oracle.decode_f64(w.q, w.key_cache, w.value_cache, kept, left.astype(np.int32), w.scale)
+    assert np.all(out[left == 0] == 0)
+    assert_attention_close(out[left > 0], ref[left > 0], f"out of pool {route} H{H} Hkv{Hkv} D{D}")
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(192, 8, 128), (136, 8, 64), (16, 16, 128)])
+@pytest.mark.parametrize("ps", [64, 0])
+def test_items_and_balanced_ranges_of_wide_head_groups(dev, H, Hkv, D, ps):
+    """G = 24 and 17 (a second head chunk of 8 and 1) and 1 in the item and the
+    balanced kernel, with empty and block-edge contexts and NaN in unused slots."""
+    rng = np.random.default_rng(H + D)
+    ctx = rng.integers(0, 90, size=140)
+    ctx[:9] = [0, 1, 15, 16, 17, 31, 33, 1100, 777]
+    w = padded(_poisoned(rng, len(ctx), ctx, D=D, H=H, Hkv=Hkv), 300)
+    assert split_route(w, ps) == ("balanced" if ps == 0 else "items")
+    out = DeviceWorkload(w).run("v2", partition_size=ps)
+    assert np.all(out[ctx == 0] == 0)
+    assert_attention_close(out, _ref(w), f"G = {H // Hkv} D{D} ps={ps}")
+
+
+@pytest.mark.parametrize("lens,list_pays", [
+    ([1500] + [600, 90, 17, 0, 1] * 30, True), ([40] * 150 + [0, 1, 1100], False), ([33] * 520 + [1100], False),
+])
+def test_single_pass_of_many_sequences_under_wide_tables(dev, lens, list_pays):
+    """v1 past three items per CU: the partition kernel, with its list where the
+    lengths call for it and in plain order where not, and past 512 sequences the
+    plain kernel."""
+    rng = np.random.default_rng(len(lens))
+    lens = np.array(lens)
+    blocks = (lens + 15) // 16
+    S = len(lens)
+    pays = S <= 512 and blocks.max() > S // 4 + 16 and blocks.sum() * 8 > 32 * S and \
+        2 * blocks.max() * S > 3 * blocks.sum()
+    assert pays == list_pays
+    w = padded(_random_batch(rng, lens, H=16, Hkv=8, D=128), 300)
+    out = DeviceWorkload(w).run("v1")
+    assert np.all(out[lens == 0] == 0)
+    assert_attention_close(out[lens > 0], _ref(w)[lens > 0], f"single pass of {S} by the list: {list_pays}")

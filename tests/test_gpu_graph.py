@@ -1,8 +1,8 @@
 """The hot path inside a HIP graph: a ragged decode step (cache write, then
-single-pass, balanced and 512-token split-K decode, the last as partition
-streams at this batch size), the fused MoE route + dispatch, and the
-whole MoE layer (MoeMlp.forward: dispatch, expert GEMMs with their thin
-tails, combine) are captured once and replayed several times, with new inputs uploaded and the
+single-pass, balanced and 512-token split-K decode: teams with 64 sequences,
+the balanced ranges and the item list with 160), the fused MoE route +
+dispatch, and the whole MoE layer (MoeMlp.forward: dispatch, expert GEMMs with
+their thin tails, combine) are captured once and replayed several times, with new inputs uploaded and the
 program's own eager work and synchronisation between replays; every replay
 must equal the eager run on the same inputs bit for bit (the kernels are
 deterministic), and the decode outputs also meet the attention tolerance."""
@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_attention_close
+from helpers import assert_attention_close, split_route
 from swiftllm_amd import moe, workloads
 from swiftllm_amd import paged_attention as pa
 from swiftllm_amd._hip import DeviceArray, Graph, Stream, synchronize
@@ -68,8 +68,10 @@ class _Step:
             dev.upload(arr)
 
 
-def test_decode_step_graph_replays_match_eager(dev):
-    w = workloads.decode_config(4, seed=31, num_seqs=64)
+@pytest.mark.parametrize("num_seqs,routes", [(64, ("teams", "teams")), (160, ("balanced", "items"))])
+def test_decode_step_graph_replays_match_eager(dev, num_seqs, routes):
+    w = workloads.decode_config(4, seed=31, num_seqs=num_seqs)
+    assert (split_route(w, 0), split_route(w, 512)) == routes
     step = _Step(w)
     stream = Stream()
     graph = Graph(stream, lambda: step.enqueue(stream))

@@ -5,7 +5,9 @@ experts, top-k) from a fixed seed, so a failure names a case that can be
 rerun exactly.
 
   decode   v1, v2 at a random partition size (multiple of 16), v2 balanced:
-           attention tolerance against oracle.decode_f64, NaN in every cache
+           attention tolerance against oracle.decode_f64 (few sequences, in a
+           single pass or by teams, and hundreds, in items and balanced
+           ranges), NaN in every cache
            slot outside the valid contexts, zero-length contexts giving zeros
   prefill  packed prompts of random lengths, positive and negative scales
            (the folded and the unfolded softmax): attention tolerance against
@@ -27,7 +29,8 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import DeviceWorkload, assert_attention_close, assert_gemm_close, expert_offsets
+from helpers import (DeviceWorkload, assert_attention_close, assert_gemm_close, expert_offsets,
+                     split_route)
 from swiftllm_amd import moe
 from swiftllm_amd import paged_attention as pa
 from swiftllm_amd import workloads
@@ -38,12 +41,13 @@ pytestmark = pytest.mark.gpu
 GQA = [(8, 8), (32, 8), (64, 8), (12, 4), (24, 2), (32, 1), (16, 1), (6, 3), (40, 8)]
 
 
-def _decode_case(seed):
+def _decode_case(seed, many=False):
+    """many: more sequences than the teams take, under tables that are split."""
     rng = np.random.default_rng(seed)
-    H, Hkv = GQA[rng.integers(len(GQA))]
+    H, Hkv = ((8, 8), (40, 8), (34, 2), (12, 4))[rng.integers(4)] if many else GQA[rng.integers(len(GQA))]
     D = int(rng.choice([64, 128]))
-    S = int(rng.integers(1, 25))
-    kind = rng.integers(3)
+    S = int(rng.integers(260, 400)) if many and Hkv > 2 else 530 if many else int(rng.integers(1, 25))
+    kind = 2 if many else rng.integers(3)
     if kind == 0:
         ctx = rng.integers(0, 2049, S)
     elif kind == 1:  # lengths on block and partition edges
@@ -75,9 +79,11 @@ def _decode_case(seed):
     return w, ps
 
 
-@pytest.mark.parametrize("seed", range(48))
+@pytest.mark.parametrize("seed", [*range(48), *range(100, 108)])
 def test_decode_random(dev, seed):
-    w, ps = _decode_case(1000 + seed)
+    w, ps = _decode_case(1000 + seed, many=seed >= 100)
+    if seed >= 100:
+        assert (split_route(w, ps), split_route(w, 0)) == ("items", "balanced")
     ref = oracle.decode_f64(w.q, w.key_cache, w.value_cache, w.block_tables, w.context_lens, w.scale)
     dw = DeviceWorkload(w)
     S, H, D = w.q.shape

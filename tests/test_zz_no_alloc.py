@@ -19,7 +19,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import assert_attention_close
+from helpers import assert_attention_close, padded, split_route
 from swiftllm_amd import _lib
 from swiftllm_amd import paged_attention as pa
 from swiftllm_amd import workloads
@@ -103,17 +103,20 @@ def test_noalloc_first_call_captured_in_a_graph(dev):
 
 
 def test_noalloc_matches_workspace_entry_on_consecutive_calls(dev):
-    """Config 3's heads at 16384 tokens in 512-token partitions (partition
-    streams: 8.4 MB of partial outputs and 8.7 MB of boundary slots in the
-    scratch, the workgroup reduce over 32 partitions), then a smaller batch
-    (config 1's shape) at 64-token partitions, then the small batch again in
-    balanced mode: each bit-equal to the workspace entry point and within the
-    oracle's tolerance."""
+    """Config 3's heads at 16384 tokens in 512-token partitions (teams: 9 MB of
+    fragments in the scratch), then smaller batches (config 1's shape): 7
+    sequences under wide tables by teams and under their own in a single pass,
+    140 under wide tables in 64-token items and balanced ranges: each bit-equal
+    to the workspace entry point and within the oracle's tolerance."""
     stream = Stream()
     big = _Case(workloads.decode_config(3, seed=31, ctx=16384))
-    small = _Case(workloads.decode_config(1, seed=32, num_seqs=7))
-    calls = [(big, 512), (small, 64), (small, 0)]
-    for case, ps in calls:
+    small = workloads.decode_config(1, seed=32, num_seqs=7)
+    many = _Case(padded(workloads.decode_config(1, seed=35, num_seqs=140), 120))
+    wide, small = _Case(padded(small, 120)), _Case(small)
+    calls = [(big, 512, "teams"), (wide, 64, "teams"), (small, 64, "single"), (small, 0, "single"),
+             (many, 64, "items"), (many, 0, "balanced")]
+    for case, ps, route in calls:
+        assert split_route(case.w, ps) == route
         got = case.noalloc(ps, stream)
         want, ws = case.with_workspace(ps, stream)
         stream.synchronize()
