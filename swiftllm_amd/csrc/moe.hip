@@ -17,7 +17,7 @@
 //           by DPP. One thread per token re-read its row from memory K times:
 //           route and dispatch of 1000 tokens over 64 experts, top-8, hidden
 //           2048, took 130 us and take 19.2; of 4096 tokens, top-6, 121 and
-//           31.5 (100 MB of rows at 5.7 TB/s of copy: 20).
+//           29.7 (100 MB of rows at 5.7 TB/s of copy: 20).
 // dispatch: two kernels, with no grid-wide synchronisation inside either.
 //           (1) rank: the entries of each 64-token chunk get their rank among
 //               equal experts (stable (t, k) order) and the chunk its counts
@@ -498,6 +498,15 @@ constexpr int kPermuteWaves = 4;       // one token per wave
 constexpr int kLdsCounts = 4096;       // count matrices up to this size are scanned in LDS
 constexpr int kLdsPad = 512;           // room for one more column (E >= 8)
 
+// Bytes of x_perm up to which its rows are stored nontemporally. Past it the
+// caches take the writes and return them in larger pieces; below it the dirty
+// lines they hold are written back at the kernel's end instead. Measured (us
+// per call, 8 experts, top-2, nontemporal / plain): 67 MB of rows 20.5 / 19.3,
+// 47.5 MB 15.3 / 15.3, 32.8 MB 11.8 / 12.9, 16.4 MB 8.6 / 9.7; 64 experts,
+// top-6, 100 MB 31.1 / 29.7. That is with the same rows written by every call;
+// with eight row sets of 67 MB in turn both take 21.3.
+constexpr size_t kNontemporalRows = 48u << 20;
+
 struct PermuteArgs {
     const int* ids;
     const int* rank;
@@ -518,18 +527,9 @@ struct PermuteArgs {
 };
 
 // VEC: rows move as 16-byte vectors (a.xp set and a.vec); otherwise index
-// arrays only, or a 2-byte copy of unaligned rows.
-//
-// The rows are stored nontemporally at every size. Plain stores only look
-// better where each call writes the same rows over again and finds them in the
-// memory-side cache (us per call, nontemporal / plain, the same rows / eight
-// sets in turn: 33.6 MB of rows, 8 experts, top-2, 11.9 / 12.8 and 12.6 / 13.4;
-// 67 MB 19.9 / 19.7 and 21.2 / 21.5; 16 experts, 67 MB, 20.8 / 20.7 and 22.4 /
-// 23.0; 64 experts, top-6, 100 MB, 31.5 / 28.4 and 31.4 / 32.5, 201 MB 51 / 43
-// and 52 / 52). A layer rewrites its rows after streaming its weights through
-// that cache, and its time does not tell the two apart (8 x 4096 x 14336, 4096
-// tokens, 2784 / 2790 us; 64 x 2048 x 1408, 711 / 713).
-template <int K, bool VEC>
+// arrays only, or a 2-byte copy of unaligned rows. NT: nontemporal stores of
+// the rows.
+template <int K, bool VEC, bool NT>
 __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const PermuteArgs a) {
     __shared__ int s_base[kLdsCounts + kLdsPad];  // [nchunks][stride] exclusive prefixes over chunks
     __shared__ int s_off[kMaxExperts];  // expert offsets
@@ -545,15 +545,6 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
     const int t = blockIdx.x * kPermuteWaves + wv;
     const bool live = t < a.T;
     const int nv = a.hidden / 8;
-    // The u-th piece of a batch, a different first one in neighbouring tokens,
-    // whose waves run in step: with all of them at the same piece of rows a
-    // power of two apart, early stores queue behind late loads. Eight row sets
-    // in turn (us per call, before / now): 8 experts, top-2, 67 MB of rows 21.4
-    // / 21.2, 134 MB 43.8 / 42.3, top-1 33.6 MB 16.6 / 15.7, 67 MB 29.8 / 28.0;
-    // 16 experts, top-2, 67 MB 22.5 / 22.1. Rows shorter than a batch gain
-    // nothing, and with six stores per load 100 MB take 34.4 instead of 31.4.
-    const int turn = (K <= 2 && nv >= 64 * kCopyBatch) ? t & (kCopyBatch - 1) : 0;
-    auto piece = [&](int u) { return (u + turn) & (kCopyBatch - 1); };
     const u32x4* __restrict__ src =
         reinterpret_cast<const u32x4*>(a.x + static_cast<size_t>(min(t, a.T - 1)) * a.hidden);
 
@@ -587,7 +578,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
     u32x4 v[kCopyBatch];
     if constexpr (VEC) {
 #pragma unroll
-        for (int u = 0; u < kCopyBatch; ++u) v[u] = __builtin_nontemporal_load(src + min(64 * piece(u) + lane, nv - 1));
+        for (int u = 0; u < kCopyBatch; ++u) v[u] = __builtin_nontemporal_load(src + min(64 * u + lane, nv - 1));
     }
 
     // Per-expert totals: from the scan kernel, or scanned here from the counts.
@@ -659,7 +650,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
             if (i0 > 0) {
 #pragma unroll
                 for (int u = 0; u < kCopyBatch; ++u) {
-                    const int i = i0 + 64 * piece(u) + lane;
+                    const int i = i0 + 64 * u + lane;
                     if (i < nv) v[u] = __builtin_nontemporal_load(src + i);
                 }
             }
@@ -669,8 +660,13 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
                 u32x4* __restrict__ dst = reinterpret_cast<u32x4*>(a.xp + rows[k] * a.hidden);
 #pragma unroll
                 for (int u = 0; u < kCopyBatch; ++u) {
-                    const int i = i0 + 64 * piece(u) + lane;
-                    if (i < nv) __builtin_nontemporal_store(v[u], dst + i);
+                    const int i = i0 + 64 * u + lane;
+                    if (i >= nv) continue;
+                    if constexpr (NT) {
+                        __builtin_nontemporal_store(v[u], dst + i);
+                    } else {
+                        dst[i] = v[u];
+                    }
                 }
             }
         }
@@ -730,8 +726,11 @@ struct PermuteLaunch {
         // are written when there are no tokens.
         const int grid = a.T > 0 ? (a.T + kPermuteWaves - 1) / kPermuteWaves : 1;
         const dim3 block(64 * kPermuteWaves);
-        if (a.xp != nullptr && a.vec) return launch(moe_permute_kernel<K, true>, dim3(grid), block, 0, s, a);
-        return launch(moe_permute_kernel<K, false>, dim3(grid), block, 0, s, a);
+        if (a.xp == nullptr || !a.vec) return launch(moe_permute_kernel<K, false, true>, dim3(grid), block, 0, s, a);
+        if (static_cast<size_t>(a.T) * K * a.hidden * sizeof(uint16_t) <= kNontemporalRows) {
+            return launch(moe_permute_kernel<K, true, true>, dim3(grid), block, 0, s, a);
+        }
+        return launch(moe_permute_kernel<K, true, false>, dim3(grid), block, 0, s, a);
     }
 };
 
