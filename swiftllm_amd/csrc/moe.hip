@@ -500,11 +500,13 @@ constexpr int kLdsPad = 512;           // room for one more column (E >= 8)
 
 // Bytes of x_perm up to which its rows are stored nontemporally. Past it the
 // caches take the writes and return them in larger pieces; below it the dirty
-// lines they hold are written back at the kernel's end instead. Measured (us
-// per call, 8 experts, top-2, nontemporal / plain): 67 MB of rows 20.5 / 19.3,
-// 47.5 MB 15.3 / 15.3, 32.8 MB 11.8 / 12.9, 16.4 MB 8.6 / 9.7; 64 experts,
-// top-6, 100 MB 31.1 / 29.7. That is with the same rows written by every call;
-// with eight row sets of 67 MB in turn both take 21.3.
+// lines they hold are written back at the kernel's end instead. Measured (us of
+// this kernel inside whole MoE layers, whose weights pass through the caches
+// between two calls, nontemporal / plain): 8 x 4096 x 14336, top-2, 16.8 MB of
+// rows 6.0 / 6.5, 33.6 MB 9.8 / 9.8, 52 MB 15.2 / 14.1, 67 MB 19.1 / 17.8; 64 x
+// 2048 x 1408, top-6, 50 MB 15.5 / 14.9, 100 MB 27.0 / 23.4. The dispatch alone,
+// rows of 67 MB, 20.4 / 19.3 per call; with eight sets of them in turn, which
+// no layer writes, 21.2 / 21.4, and 64 experts, 100 MB, 31.4 / 32.4.
 constexpr size_t kNontemporalRows = 48u << 20;
 
 struct PermuteArgs {
@@ -545,6 +547,16 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
     const int t = blockIdx.x * kPermuteWaves + wv;
     const bool live = t < a.T;
     const int nv = a.hidden / 8;
+    // The u-th piece of a batch, a different first one in neighbouring tokens,
+    // whose waves run in step: with all of them at the same piece of rows a
+    // power of two apart, early stores queue behind late loads. Eight row sets
+    // in turn (us per dispatch, before / now): 16 experts, top-2, 67 MB of rows
+    // 23.0 / 22.5, 134 MB 43.5 / 42.7; 8 experts, top-1, 33.6 MB 16.5 / 15.8, 67
+    // MB 30.1 / 29.1, top-2, 67 MB 21.4 / 21.4; in a layer 16.8 / 16.7. Rows
+    // shorter than a batch gain nothing, and with six stores a load 100 MB took
+    // 35.7 instead of 32.6.
+    const int turn = (K <= 2 && nv >= 64 * kCopyBatch) ? t & (kCopyBatch - 1) : 0;
+    auto piece = [&](int u) { return (u + turn) & (kCopyBatch - 1); };
     const u32x4* __restrict__ src =
         reinterpret_cast<const u32x4*>(a.x + static_cast<size_t>(min(t, a.T - 1)) * a.hidden);
 
@@ -578,7 +590,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
     u32x4 v[kCopyBatch];
     if constexpr (VEC) {
 #pragma unroll
-        for (int u = 0; u < kCopyBatch; ++u) v[u] = __builtin_nontemporal_load(src + min(64 * u + lane, nv - 1));
+        for (int u = 0; u < kCopyBatch; ++u) v[u] = __builtin_nontemporal_load(src + min(64 * piece(u) + lane, nv - 1));
     }
 
     // Per-expert totals: from the scan kernel, or scanned here from the counts.
@@ -650,7 +662,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
             if (i0 > 0) {
 #pragma unroll
                 for (int u = 0; u < kCopyBatch; ++u) {
-                    const int i = i0 + 64 * u + lane;
+                    const int i = i0 + 64 * piece(u) + lane;
                     if (i < nv) v[u] = __builtin_nontemporal_load(src + i);
                 }
             }
@@ -660,7 +672,7 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void moe_permute_kernel(const P
                 u32x4* __restrict__ dst = reinterpret_cast<u32x4*>(a.xp + rows[k] * a.hidden);
 #pragma unroll
                 for (int u = 0; u < kCopyBatch; ++u) {
-                    const int i = i0 + 64 * u + lane;
+                    const int i = i0 + 64 * piece(u) + lane;
                     if (i >= nv) continue;
                     if constexpr (NT) {
                         __builtin_nontemporal_store(v[u], dst + i);
