@@ -49,7 +49,7 @@ def test_many_short_prompts(dev, S, L, H, Hkv, D):
     us = [best_us(lambda stream: pa.launch_paged_prefill(out, q, kc, vc, sm, ctx, sign / np.sqrt(D), S, H, Hkv, D,
                                                          16, L, num_blocks=NB, stream=stream))
           for sign in (1, -1)]
-    assert us[0] < 1.12 * us[1], f"{us[0]:.1f} us, per wave {us[1]:.1f} us"
+    assert us[0] < 1.15 * us[1], f"{us[0]:.1f} us, per wave {us[1]:.1f} us"
 
 
 @pytest.mark.parametrize("Hkv,D", [(2, 128), (1, 128)])
@@ -117,7 +117,7 @@ def test_single_pass_of_short_contexts_under_wide_tables(dev, S, H, Hkv, D):
     against 9.3, 65 against 28)."""
     lens = np.random.default_rng(S).integers(16, 129, size=S)
     us = [best_us(_Decode(lens, H, Hkv, D, blocks).v1) for blocks in (512, 8)]
-    assert us[0] < 1.4 * us[1], f"{us[0]:.1f} us, tables of 8 blocks {us[1]:.1f} us"
+    assert us[0] < 1.5 * us[1], f"{us[0]:.1f} us, tables of 8 blocks {us[1]:.1f} us"
 
 
 @pytest.mark.parametrize("S", [64, 96])
